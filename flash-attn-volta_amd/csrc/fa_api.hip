@@ -503,27 +503,103 @@ struct SplitPlan {
   int kv_split;   // keys per split, a multiple of the 64-key tile
 };
 
-// Split when one packed 64-row tile holds a key/value head's whole group of
-// query rows (grp * Sq <= 64), the regular grid would leave the GPU
-// under-filled, and there are enough keys: about 2 workgroups per CU, at
-// least 128 keys per split (measured against 4 and 8 per CU and a 64- or
-// 256-key minimum: equal or faster on every decode shape of bench.py).
+// Packed rows (query position, head of the group) of one key/value head, and
+// the 64-row tiles of them over all (b, key/value head): the workgroups of
+// one key range.
+int64_t packed_tiles(const Shape &s) {
+  const int64_t rows = (int64_t)(s.H / s.Hk) * s.Sq;
+  return (rows + 63) / 64 * s.B * s.Hk;
+}
+
+SplitPlan split_of(const Shape &s, int64_t n) {
+  const int64_t kv = ((s.Sk + n - 1) / n + 63) / 64 * 64;
+  n = (s.Sk + kv - 1) / kv;
+  if (n < 2 || n > 65535) return SplitPlan{0, 0};
+  return SplitPlan{(int)n, (int)kv};
+}
+
+// Decode: one packed tile holds a key/value head's whole group of query
+// rows (grp * Sq <= 64), so the time is streaming K and V once.  Two
+// workgroups run per CU; n ranges of at least 128 keys (measured against a
+// 64- or 256-key minimum: equal or faster on every decode shape of
+// bench.py), n the count with the fewest rounds times (tiles per range + 3,
+// a workgroup's start-up).
+SplitPlan decode_split(const Shape &s) {
+  const int64_t slots = 2 * (int64_t)device_cus(), heads = (int64_t)s.B * s.Hk;
+  const int64_t max_n = (s.Sk + 127) / 128;
+  int64_t best = 1, cost = 0;
+  // the counts that just fill 1 .. 8 rounds (between them only rounds grow)
+  for (int64_t k = 1; k <= 8; ++k) {
+    int64_t n = k * slots / heads;
+    n = n < 1 ? 1 : (n > max_n ? max_n : n);
+    const int64_t c = (heads * n + slots - 1) / slots * ((s.Sk + 64 * n - 1) / (64 * n) + 3);
+    if (k == 1 || c < cost) {
+      best = n;
+      cost = c;
+    }
+  }
+  return split_of(s, best);
+}
+
 SplitPlan splitkv_plan(const Shape &s) {
   const SplitPlan none{0, 0};
   const int64_t grp = s.H / s.Hk;
   if (grp * s.Sq > 64 || s.Sk < 256) return none;
+  if ((int64_t)((s.Sq + 63) / 64) * s.B * s.H >= 2 * (int64_t)device_cus()) return none;
+  return decode_split(s);
+}
+
+// fa_fwd_ws's key split: splitkv_plan's, and
+//   * decode with grouped heads whose plain grid does fill the GPU: the
+//     plain grid reads K and V once per query head, the packed tile once
+//     ((32, 1, 3001 keys, 32 heads / 8, 128) bf16: 222 us plain, 74 us
+//     packed, 5.3 TB/s, a large copy's rate; (64, 4, 4000, 32 / 8, 128)
+//     595 -> 179 us);
+//   * chunks: any short block of queries whose plain grid leaves CUs idle.
+//     The model below prices both: a CU runs one 64 x 64 tile step in `step`
+//     us whether one workgroup or two share it, a packed launch adds about
+//     8 us of start-up and merge and the partials' traffic.  Measured, bf16
+//     (1, Sq, 8448 keys, 32 / 8, 128): Sq = 256 90 -> 52 us, 128 92 -> 32,
+//     32 92 -> 19; from Sq = 512 on (one plain workgroup per CU) splitting
+//     gains nothing and the model keeps the plain grid.
+SplitPlan fwd_split_plan(const Shape &s, int causal) {
+  const SplitPlan none{0, 0};
+  const int64_t grp = s.H / s.Hk;
+  if (s.Sk < 256) return none;
   const int64_t cus = device_cus();
-  const int64_t regular = (int64_t)((s.Sq + 63) / 64) * s.B * s.H;
-  if (regular >= 2 * cus) return none;
-  const int64_t heads = (int64_t)s.B * s.Hk;
-  int64_t n = (2 * cus + heads - 1) / heads;
-  const int64_t max_n = (s.Sk + 127) / 128;
-  if (n > max_n) n = max_n;
-  if (n < 2) return none;
-  const int64_t kv = ((s.Sk + n - 1) / n + 63) / 64 * 64;
-  n = (s.Sk + kv - 1) / kv;
-  if (n < 2 || n > 65535) return none;
-  return SplitPlan{(int)n, (int)kv};
+  const int64_t plain = (int64_t)((s.Sq + 63) / 64) * s.B * s.H;
+  if (grp * s.Sq <= 64) {
+    if (plain >= 2 * cus && grp == 1) return none;
+    return decode_split(s);
+  }
+  // (a causal grid's plain sweeps must be near the full length: at least
+  // half of the keys lie before the block)
+  if (causal && (int64_t)s.Sk < 2 * (int64_t)s.Sq) return none;
+  const double step = s.D >= 128 ? 0.6 : 0.35;
+  const int64_t tiles = (s.Sk + 63) / 64, packed = packed_tiles(s);
+  const double t_plain = (double)((plain + cus - 1) / cus) * tiles * step;
+  double best = 0.85 * t_plain;
+  int64_t best_n = 0;
+  for (int64_t k = 1; k <= 8; ++k) {
+    const int64_t n = k * cus / packed < tiles / 4 ? k * cus / packed : tiles / 4;
+    if (n < 2) continue;
+    const int64_t t = (tiles + n - 1) / n;
+    const double rows = (double)s.B * s.H * s.Sq * n;
+    const double c = (double)((packed * n + cus - 1) / cus) * t * step + 8.0 +
+                     rows * (s.D + 1) * 8.0 / 5.0e6;
+    if (c < best) {
+      best = c;
+      best_n = n;
+    }
+  }
+  return best_n ? split_of(s, best_n) : none;
+}
+
+// The packed tile as one key range, written directly (no workspace): decode
+// with grouped heads on grids of at least one packed tile per CU.
+bool packed_direct(const Shape &s) {
+  const int64_t grp = s.H / s.Hk;
+  return grp > 1 && grp * s.Sq <= 64 && packed_tiles(s) >= device_cus();
 }
 
 // Workspace: part_o (n_splits, B, H, Sq, D) fp32, then part_lse (n_splits, B, H, Sq) fp32.
@@ -562,7 +638,7 @@ int launch_fwd_splitkv(const SplitLaunch &L, hipStream_t stream) {
                        dim3((unsigned)gx, L.n_splits), dim3(T::NT), 0, stream, a);
   }
   int rc = launch_status();
-  if (rc) return rc;
+  if (rc || L.n_splits == 1) return rc;   // one range: O is written
   const int64_t rows = (int64_t)a.B * a.H * a.Sq;
   fa::CombineArgs c = L.c;
   constexpr int SLOTS = 256 / (D / 8);
@@ -621,17 +697,24 @@ int run_fwd(const void *q, const void *k, const void *v, void *o, float *lse, co
   if (rc) return rc;
   const fa::FwdArgs a = fwd_args(q, k, v, o, lse, s, q_st, k_st, v_st, o_st, sm_scale);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (packed_direct(s)) {
+    SplitLaunch L{};
+    L.f = a;
+    L.f.kv_split = s.Sk;
+    L.n_splits = 1;
+    FA_DISPATCH(launch_fwd_splitkv, s, causal, L, st);
+  }
   FA_DISPATCH(launch_fwd, s, causal, a, st);
 }
 
 int run_fwd_splitkv(const void *q, const void *k, const void *v, void *o, float *lse,
                     void *workspace, size_t workspace_bytes, const Shape &s, const int64_t *q_st,
                     const int64_t *k_st, const int64_t *v_st, const int64_t *o_st, float sm_scale,
-                    int causal, void *stream) {
+                    int causal, bool chunks, void *stream) {
   const LaunchDevice launch_dev(stream);
   int rc = check_fwd(q, k, v, o, lse, s, q_st, k_st, v_st, o_st, sm_scale);
   if (rc) return rc;
-  const SplitPlan plan = splitkv_plan(s);
+  const SplitPlan plan = chunks ? fwd_split_plan(s, causal) : splitkv_plan(s);
   if (plan.n_splits == 0)
     return run_fwd(q, k, v, o, lse, s, q_st, k_st, v_st, o_st, sm_scale, causal, stream);
   if (workspace == nullptr || workspace_bytes < splitkv_bytes(s, plan)) return FA_ERR_WORKSPACE;
@@ -757,7 +840,7 @@ int launch_fwd_bal(const BalLaunch &L, hipStream_t stream) {
 }
 
 size_t fwd_ws_bytes(const Shape &s, int causal) {
-  const SplitPlan kv = splitkv_plan(s);
+  const SplitPlan kv = fwd_split_plan(s, causal);
   if (kv.n_splits) return splitkv_bytes(s, kv);
   return bal_bytes(s, bal_plan(s, causal));
 }
@@ -774,9 +857,9 @@ int run_fwd_ws(const void *q, const void *k, const void *v, void *o, float *lse,
   if (need == 0 || workspace == nullptr || workspace_bytes < need)
     return run_fwd(q, k, v, o, lse, s, q_st, k_st, v_st, o_st, sm_scale, causal, stream);
   if (!aligned16(workspace)) return FA_ERR_ALIGNMENT;
-  if (splitkv_plan(s).n_splits)
+  if (fwd_split_plan(s, causal).n_splits)
     return run_fwd_splitkv(q, k, v, o, lse, workspace, workspace_bytes, s, q_st, k_st, v_st, o_st,
-                           sm_scale, causal, stream);
+                           sm_scale, causal, true, stream);
   const BalPlan plan = bal_plan(s, causal);
   if (plan.nb == 0)
     return run_fwd(q, k, v, o, lse, s, q_st, k_st, v_st, o_st, sm_scale, causal, stream);
@@ -1620,7 +1703,7 @@ int fa_fwd_splitkv(const void *q, const void *k, const void *v, void *o, float *
                    float sm_scale, int causal, int dtype, void *stream) {
   return run_fwd_splitkv(q, k, v, o, lse, workspace, workspace_bytes,
                          Shape{B, Sq, Sk, H, Hk, D, dtype}, q_strides, k_strides, v_strides,
-                         o_strides, sm_scale, causal, stream);
+                         o_strides, sm_scale, causal, false, stream);
 }
 
 size_t fa_fwd_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, int causal) {

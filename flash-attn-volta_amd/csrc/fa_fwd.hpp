@@ -60,7 +60,7 @@ struct FwdArgs {
   int zigzag;          // causal tile order: 1 zigzag heavy / light, 0 heaviest first
   // split-KV mode only (fa_fwd_kernel<..., SPLITKV = true>):
   int kv_split;        // keys per split, a multiple of the 64-key tile
-  float *part_o;       // (n_splits, B, H, Sq, D) fp32: each split's normalised O
+  float *part_o;       // (n_splits, B, H, Sq, D) fp32: each split's normalised O; NULL: one split, O itself
   float *part_lse;     // (n_splits, B, H, Sq) fp32: each split's LSE in log2 units
   // The balanced causal mode (BAL = true) writes its split tiles' halves to
   // part_o / part_lse as (2, B, H, n_qtiles / 2, BM, D) and (2, B, H,
@@ -176,12 +176,13 @@ struct FwdTile {
 // causal attention, whose last query tile walks every key tile.  The
 // launcher picks KSPLIT from the grid size.
 //
-// SPLITKV (decode against a long cache): the rows of a tile are the
+// SPLITKV (a short block of queries against long keys): the rows are the
 // (query position, query head) pairs of one key/value head's group, row
 // r = position * grp + head-in-group, so the group's heads share each K/V
 // tile; blockIdx.y selects a range of kv_split keys, and the workgroup
 // writes its rows' normalised O and log2-domain LSE over that range to
-// part_o / part_lse, which fa_fwd_combine_kernel merges.
+// part_o / part_lse, which fa_fwd_combine_kernel merges -- or, with one
+// range (part_o NULL), O and LSE themselves.
 template <typename E, int D, bool CAUSAL, int KSPLIT, bool SPLITKV = false, bool PRE = false,
           bool BAL = false, int NW = 4>
 __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
@@ -776,13 +777,14 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
   // ---- epilogue: O = acc / l, LSE = (m + log2 l) * ln2
   const float l_tot = l_run + xor32(l_run);
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  if (SPLITKV || (BAL && part >= 0)) {
+  // SPLITKV: the lane's query head
+  const int hq = SPLITKV ? hk * grp + qrow % grp : h;
+  if ((SPLITKV && a.part_o != nullptr) || (BAL && part >= 0)) {
     // this split's normalised O and log2-domain LSE (-inf: no visible key)
     if (qrow < nrows) {
       int64_t prow;
       if (SPLITKV) {
-        const int hq = hk * grp + qrow % grp;
-        prow = (((int64_t)blockIdx.y * a.B + b) * a.H + hq) * Sq + qrow / grp;
+        prow = (((int64_t)blockIdx.y * a.B + b) * a.H + hq) * Sq + qpos;
       } else {
         // (half, slot (b, h, pair), row in the tile)
         const int64_t rows = (int64_t)BH * (a.n_qtiles >> 1) * BM;
@@ -803,8 +805,8 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
     }
     return;
   }
-  if (qrow < Sq) {
-    f16 *orow = a.o + b * a.o_sb + h * a.o_sh + (int64_t)qrow * a.o_ss;
+  if (qrow < nrows) {
+    f16 *orow = a.o + b * a.o_sb + hq * a.o_sh + (int64_t)qpos * a.o_ss;
 #pragma unroll
     for (int d = 0; d < D / 32; ++d) {
 #pragma unroll
@@ -817,7 +819,7 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
     }
     if (a.lse != nullptr && g == 0) {
       const float lse = l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2 : kPosInf;
-      a.lse[(int64_t)bh * Sq + qrow] = lse;
+      a.lse[((int64_t)b * a.H + hq) * Sq + qpos] = lse;
     }
   }
 }

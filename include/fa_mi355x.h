@@ -106,6 +106,9 @@ int fa_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
  * q, k, v and o; accumulation is fp32 either way.  With Sq == Sk, Hk == H
  * and FA_DTYPE_F16 it is fa_fwd.
  *
+ * With grouped heads and H / Hk * Sq <= 64, on grids of at least one
+ * key/value head per compute unit, the heads of a group share one tile.
+ *
  * No counterpart in the reference kernels, whose wrapper asserts equal
  * q/k/v shapes (flash_attn_volta/triton_fa.py:315); it replaces the
  * repeat_kv expansion of K/V the reference's HuggingFace patch does before
@@ -150,7 +153,10 @@ size_t fa_fwd_splitkv_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int 
  * Forward with a workspace: the schedule that is fastest for these sizes.
  * Same arguments and results as fa_fwd_gqa (to fp32 rounding of a merge),
  * plus `workspace`, `workspace_bytes`.
- *   - Short query blocks against long keys: fa_fwd_splitkv's key split.
+ *   - Short query blocks against long keys: the key split of fa_fwd_splitkv,
+ *     here also for query blocks of several packed tiles (H / Hk * Sq > 64)
+ *     whose plain grid leaves compute units idle, and for grouped heads
+ *     whose plain grid fills the GPU.
  *   - Causal, Sq == Sk, at least 32 query tiles of 64 rows per head and at
  *     most half a tile per compute unit in the plain grid (one from 48
  *     tiles per head, 1.75 from 64): query tiles paired
