@@ -328,13 +328,23 @@ int launch_pre(const fa::PreArgs &a, hipStream_t stream) {
   return launch_status();
 }
 
+// Sums the segments of a dK/dV launch (BwdArgs::seg_n > 1).
+template <typename E, int D>
+int launch_seg_sum(const fa::BwdArgs &a, hipStream_t stream) {
+  const int64_t grid = ((int64_t)a.B * a.Hk * a.Sk * (D / 4) + 255) / 256;
+  if (grid > 0x7fffffff) return FA_ERR_TOO_LARGE;
+  hipLaunchKernelGGL((fa::fa_bwd_seg_sum_kernel<E, D>), dim3((unsigned)grid, 2), dim3(256), 0,
+                     stream, a);
+  return launch_status();
+}
+
 template <typename E, int D, bool CAUSAL, int SPLIT>
 int launch_dkdv_split(const fa::BwdArgs &args, hipStream_t stream) {
   using T = fa::DkdvTile<D, SPLIT>;
   fa::BwdArgs a = args;
   a.n_blocks = (a.Sk + T::BK - 1) / T::BK;
-  // a split key block takes two workgroups
-  const int64_t grid = ((int64_t)a.n_blocks + a.split_kt) * a.B * a.Hk;
+  // a split key block takes two workgroups, one in segments seg_n
+  const int64_t grid = ((int64_t)a.n_blocks * a.seg_n + a.split_kt) * a.B * a.Hk;
   if (grid > 0x7fffffff) return FA_ERR_TOO_LARGE;
   constexpr auto kernel = fa::fa_bwd_dkdv_kernel<E, D, CAUSAL, SPLIT>;
   // Causal order (unsplit grids): heaviest first, except zigzag heavy /
@@ -343,14 +353,15 @@ int launch_dkdv_split(const fa::BwdArgs &args, hipStream_t stream) {
   // zigzag -3 % at (1,4096,16,64) (1.33 rounds), -1.4 % at (1,3072,16,64);
   // heaviest first -5 % at (1,2048,32,64) (32 blocks per head), -10 % at
   // (1,4096,32,64) (2.67 rounds), -17 % on the D = 128 grids.
-  if (CAUSAL && a.split_kt == 0 && a.n_blocks >= 48) {
+  if (CAUSAL && a.split_kt == 0 && a.seg_n == 1 && a.n_blocks >= 48) {
     const int per_cu = resident_per_cu<kernel>(T::NT);
     a.zigzag = per_cu > 0 && 2 * grid <= 3 * (int64_t)per_cu * device_cus() ? 1 : 0;
   } else {
     a.zigzag = 0;
   }
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(T::NT), 0, stream, a);
-  return launch_status();
+  const int rc = launch_status();
+  return rc || a.seg_n == 1 ? rc : launch_seg_sum<E, D>(a, stream);
 }
 
 template <typename E, int D, bool CAUSAL, int SPLIT, bool PRE, int NW = 4>
@@ -380,7 +391,7 @@ int launch_dkdv(const fa::BwdArgs &a, hipStream_t stream) {
   if constexpr (D == 64 && CAUSAL) {
     if (a.split_kt > 0) return launch_dkdv_split<E, D, CAUSAL, 2>(a, stream);
   }
-  return row_split(a.Sk, (int64_t)a.B * a.Hk, CAUSAL, D >= 128 ? 1 : 2)
+  return row_split(a.Sk, (int64_t)a.B * a.Hk * a.seg_n, CAUSAL, D >= 128 ? 1 : 2)
              ? launch_dkdv_split<E, D, CAUSAL, 2>(a, stream)
              : launch_dkdv_split<E, D, CAUSAL, 1>(a, stream);
 }
@@ -436,7 +447,8 @@ int launch_bwd_fused_as(FusedBwd f, hipStream_t stream) {
   using Q = fa::DqTile<D, QS, T::NW>;
   f.akv.n_blocks = (f.akv.Sk + T::BK - 1) / T::BK;
   f.aq.n_blocks = (f.aq.Sq + Q::BM - 1) / Q::BM;
-  const int64_t n_kv = ((int64_t)f.akv.n_blocks + f.akv.split_kt) * f.akv.B * f.akv.Hk;
+  const int64_t n_kv =
+      ((int64_t)f.akv.n_blocks * f.akv.seg_n + f.akv.split_kt) * f.akv.B * f.akv.Hk;
   const int64_t n_q = (int64_t)f.aq.n_blocks * f.aq.B * f.aq.H;
   if (n_kv + n_q > 0x7fffffff) return FA_ERR_TOO_LARGE;
   // heaviest blocks first in both parts: the last workgroups dispatched
@@ -447,16 +459,16 @@ int launch_bwd_fused_as(FusedBwd f, hipStream_t stream) {
     const int rc = launch_pre<E, D>(f.pre, stream);
     if (rc) return rc;
   }
-  if constexpr (std::is_same<E, fa::f16>::value) {
-    if (f.aq.c <= 1.0f) {
-      hipLaunchKernelGGL((fa::fa_bwd_fused_kernel<E, D, CAUSAL, KVS, QS, true>),
-                         dim3((unsigned)(n_kv + n_q)), dim3(T::NT), 0, stream, f.akv, f.aq, (int)n_kv);
-      return launch_status();
-    }
-  }
-  hipLaunchKernelGGL((fa::fa_bwd_fused_kernel<E, D, CAUSAL, KVS, QS, false>),
-                     dim3((unsigned)(n_kv + n_q)), dim3(T::NT), 0, stream, f.akv, f.aq, (int)n_kv);
-  return launch_status();
+  const dim3 grid((unsigned)(n_kv + n_q));
+  constexpr bool F16 = std::is_same<E, fa::f16>::value;
+  if (F16 && f.aq.c <= 1.0f)
+    hipLaunchKernelGGL((fa::fa_bwd_fused_kernel<E, D, CAUSAL, KVS, QS, F16>), grid, dim3(T::NT), 0,
+                       stream, f.akv, f.aq, (int)n_kv);
+  else
+    hipLaunchKernelGGL((fa::fa_bwd_fused_kernel<E, D, CAUSAL, KVS, QS, false>), grid, dim3(T::NT),
+                       0, stream, f.akv, f.aq, (int)n_kv);
+  const int rc = launch_status();
+  return rc || f.akv.seg_n == 1 ? rc : launch_seg_sum<E, D>(f.akv, stream);
 }
 
 template <typename E, int D, bool CAUSAL>
@@ -951,6 +963,7 @@ int bwd_common(const void *dout, const void *q, const void *k, const void *v, co
   a.lse_mul = lse_seed_mul(a.c, s.dtype);
   a.sm_scale = sm_scale;
   a.neg = sm_scale < 0.0f;
+  a.seg_n = 1;
   *out = a;
   return FA_OK;
 }
@@ -1094,11 +1107,11 @@ DqSplit dq_split_plan(const Shape &s, int causal) {
 //   (2,4096,4,128) -9.7 % -- the dQ blocks fill the slots the unequal
 //   sweeps leave idle, as the split's second workgroups did, without its
 //   partials.
-bool bwd_fused(const Shape &s, int causal, const DqSplit &qplan) {
+bool bwd_fused(const Shape &s, int causal, const DqSplit &qplan, int seg_n = 1) {
   if (!causal || qplan.split != 0) return false;
   if (s.D <= 64) return true;
   using T = fa::DkdvTile<128, 1>;
-  const int64_t blocks = (s.Sk + T::BK - 1) / T::BK * ((int64_t)s.B * s.Hk);
+  const int64_t blocks = (s.Sk + T::BK - 1) / T::BK * ((int64_t)s.B * s.Hk) * seg_n;
   return blocks <= 4 * (int64_t)device_cus();
 }
 
@@ -1119,6 +1132,60 @@ void bwd_plans(const Shape &s, int causal, DkdvSplit &plan, DqSplit &qplan) {
   if (qplan.split != 0 && qplan.sweep < min_sweep && bwd_fused(s, causal, DqSplit{}))
     qplan = DqSplit{};
   plan = bwd_fused(s, causal, qplan) ? DkdvSplit{} : dkdv_split_plan(s, causal);
+}
+
+// Sweep segments of the dK/dV blocks (fa::BwdArgs::seg_n), given the room
+// (fa_bwd_best_workspace_bytes).  A key block's sweep covers every query
+// head of its group, so few key/value heads leave few, long workgroups:
+// (1, 4000, 28 heads / 4, 128) causal is 128 workgroups of up to 441 query
+// tiles on 256 CUs.  A segment costs its fp32 rows (written once, read once
+// by the sum) and a workgroup's start-up, so as few as fill the GPU.
+// Measured, the backward (1 segment -> chosen), causal, D = 128:
+//   (1,4000,28/4) 762 -> 444 us (2; 4: 444, 8: 469), (1,3000,28/4) 563 -> 272
+//   (3), (1,2048,16/2) 428 -> 91 (8), (1,1024,32/8) 121 -> 62 (4),
+//   (1,512,32/8) 67 -> 40 (3), (1,3500,32/8) 411 -> 388 (2), (1,4096,32/8)
+//   (one full round, 256-tile sweeps) 510 -> 487 (2), but (1,4096,16/8) (one
+//   round, 128 tiles) +6 % and (2,3000,16/8) (1.5 rounds) +11 % with 2;
+// D = 64: (1,4096,14/2) 396 -> 134 (8), (1,2048,32/8) 131 -> 89 (4);
+// equal heads: (1,2048,4/4) 65 -> 55, (2,1500,4/4) 54 -> 48 (2), but
+//   (1,2048,8/8) +6 %;
+// not causal: (1,2048,32/4,128) 467 -> 254 (4), (1,3000,32/8,128) 754 -> 529
+//   (4), (1,4096,4/4,128) 161 -> 149 (2), (1,4096,14/2,64) 470 -> 245 (8), but
+//   (2,1024,8/8,64) (16-tile sweeps) +24 % with 2.
+int dkdv_segments(const Shape &s, int causal) {
+  const int64_t grp = s.H / s.Hk;
+  const int64_t blocks = (int64_t)((s.Sk + 127) / 128) * s.B * s.Hk;
+  const int64_t slots = (s.D >= 128 ? 1 : 2) * (int64_t)device_cus();
+  const int64_t sweep = causal ? causal_tiles(s, 0, 128, 64) : (int64_t)((s.Sq + 63) / 64) * grp;
+  if (!causal) {
+    // rounds times (tiles of a segment + 3, a workgroup's start-up), at
+    // least 16 tiles each; 10 % better at least
+    int64_t best = 1, cost = (blocks + slots - 1) / slots * (sweep + 3) * 9 / 10;
+    for (int64_t n = 2; n <= 16 && 16 * n <= sweep; ++n) {
+      const int64_t c = (blocks * n + slots - 1) / slots * ((sweep + n - 1) / n + 3);
+      if (c < cost) {
+        best = n;
+        cost = c;
+      }
+    }
+    return (int)best;
+  }
+  if (grp == 1) {
+    DkdvSplit plan;
+    DqSplit qplan;
+    bwd_plans(s, causal, plan, qplan);
+    return s.D == 128 && 8 * blocks <= 3 * slots && sweep >= 20 && qplan.split == 0 ? 2 : 1;
+  }
+  if (blocks > slots) return 1;
+  int64_t n = (slots + blocks - 1) / blocks;
+  if (n < 2 && sweep >= 192) n = 2;
+  if (n > sweep / 10) n = sweep / 10;
+  return n < 2 ? 1 : (n > 16 ? 16 : (int)n);
+}
+
+// one segment's fp32 dK and dV
+size_t segment_bytes(const Shape &s) {
+  return (size_t)2 * s.B * s.Hk * (size_t)s.Sk * s.D * sizeof(float);
 }
 
 // two segments x BM rows x D fp32 per split query block
@@ -1184,12 +1251,15 @@ int run_dkdv(const void *dout, const void *q, const void *k, const void *v, cons
              const int64_t *q_st, const int64_t *k_st, const int64_t *v_st, const int64_t *dk_st,
              const int64_t *dv_st, float sm_scale, int causal, void *stream, int split_kt = 0,
              unsigned *cnt = nullptr, float *part = nullptr, const DqSplit *dqs = nullptr,
-             float *dq_part = nullptr, void *dq = nullptr, const int64_t *dq_st = nullptr) {
+             float *dq_part = nullptr, void *dq = nullptr, const int64_t *dq_st = nullptr,
+             int seg_n = 1, float *seg_part = nullptr) {
   const LaunchDevice launch_dev(stream);
   fa::BwdArgs a;
   int rc = dkdv_args(dout, q, k, v, lse, delta, rmax, dk, dv, s, do_st, q_st, k_st, v_st, dk_st,
                      dv_st, sm_scale, split_kt, cnt, part, dqs, dq_part, dq, dq_st, &a);
   if (rc) return rc;
+  a.seg_n = seg_n;
+  a.seg_part = seg_part;
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_dkdv, s, causal, a, st);
 }
@@ -1290,7 +1360,11 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
   float *rmax = reinterpret_cast<float *>(static_cast<char *>(workspace) +
                                           delta_bytes(s.B, s.Sq, s.H));
   const size_t dbytes = delta_bytes(s.B, s.Sq, s.H) + rbytes;
-  if (workspace_bytes < dbytes + split_bytes(plan) + dq_split_bytes(qplan)) {
+  // Sweep segments where the workspace has room for all of them
+  // (fa_bwd_best_workspace_bytes), in place of both splits.
+  int seg_n = dkdv_segments(s, causal);
+  if (workspace_bytes < dbytes + seg_n * segment_bytes(s)) seg_n = 1;
+  if (seg_n > 1 || workspace_bytes < dbytes + split_bytes(plan) + dq_split_bytes(qplan)) {
     plan = DkdvSplit{};
     qplan = DqSplit{};
   }
@@ -1303,7 +1377,9 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
   }
   float *dq_part =
       qplan.split > 0 ? reinterpret_cast<float *>(ws + dbytes + split_bytes(plan)) : nullptr;
-  if (bwd_fused(s, causal, qplan)) {
+  // the segments' partials follow delta and the maxima
+  float *seg_part = reinterpret_cast<float *>(ws + dbytes);
+  if (bwd_fused(s, causal, qplan, seg_n)) {
     FusedBwd f{};
     if ((rc = dkdv_args(dout, q, k, v, lse, delta, rmax, dk, dv, s, do_st, q_st, k_st, v_st,
                         dk_st, dv_st, sm_scale, plan.split_kt, cnt, part, nullptr, nullptr,
@@ -1322,7 +1398,9 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
     f.pre.cnt_zero = cnt;
     f.pre.n_cnt_zero = (int)plan.slots;
     f.with_pre = true;
-    f.kv_split2 = plan.split_kt > 0 || row_split(s.Sk, (int64_t)s.B * s.Hk, true, 2);
+    f.akv.seg_n = seg_n;
+    f.akv.seg_part = seg_part;
+    f.kv_split2 = plan.split_kt > 0 || row_split(s.Sk, (int64_t)s.B * s.Hk * seg_n, true, 2);
     f.q_split2 = row_split(s.Sq, (int64_t)s.B * s.H, true);
     hipStream_t st = static_cast<hipStream_t>(stream);
     FA_DISPATCH(launch_bwd_fused, s, causal, f, st);
@@ -1336,7 +1414,7 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
     return rc;
   return run_dkdv(dout, q, k, v, lse, delta, rmax, dk, dv, s, do_st, q_st, k_st, v_st, dk_st,
                   dv_st, sm_scale, causal, stream, plan.split_kt, cnt, part, &qplan, dq_part, dq,
-                  dq_st);
+                  dq_st, seg_n, seg_part);
 }
 
 // Both gradient launches given delta (fa_bwd without its delta step):
@@ -1748,6 +1826,14 @@ size_t fa_bwd_gqa_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, i
   return delta_bytes(B, Sq, H) + rmax_bytes(B, Sq, H) + split_bytes(plan) + dq_split_bytes(qplan);
 }
 
+size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, int causal) {
+  const Shape s{B, Sq, Sk, H, Hk, D, FA_DTYPE_F16};
+  if (check_shape(s) != FA_OK) return 0;
+  const int seg_n = dkdv_segments(s, causal);
+  if (seg_n == 1) return fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, causal);
+  return delta_bytes(B, Sq, H) + rmax_bytes(B, Sq, H) + seg_n * segment_bytes(s);
+}
+
 int fa_bwd(const void *dout, const void *q, const void *k, const void *v,
            const void *o, const float *lse,
            void *dq, void *dk, void *dv,
@@ -1795,8 +1881,11 @@ int fa_bwd_gqa_noalloc(const void *dout, const void *q, const void *k, const voi
     return FA_ERR_SCRATCH;
   void *ws = nullptr;
   if ((rc = scratch_for_stream(stream, &ws))) return rc;
-  return run_bwd(dout, q, k, v, o, lse, dq, dk, dv, ws, FA_NOALLOC_SCRATCH_BYTES, s, do_strides,
-                 q_strides, k_strides, v_strides, o_strides, dq_strides, dk_strides, dv_strides,
+  // (the splits as fa_bwd_gqa with this size; no sweep segments)
+  const size_t most = fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, causal);
+  return run_bwd(dout, q, k, v, o, lse, dq, dk, dv, ws,
+                 most < FA_NOALLOC_SCRATCH_BYTES ? most : (size_t)FA_NOALLOC_SCRATCH_BYTES, s,
+                 do_strides, q_strides, k_strides, v_strides, o_strides, dq_strides, dk_strides, dv_strides,
                  sm_scale, causal, stream);
 }
 

@@ -135,6 +135,13 @@ struct BwdArgs {
   int split_kt;
   unsigned *cnt;
   float *part;
+  // Sweep segments of the dK/dV blocks: with seg_n > 1 every key block is
+  // swept by seg_n workgroups, each taking an equal run of the block's
+  // flattened (query head of the group, query tile) list and writing its
+  // fp32 dK / dV rows to seg_part (seg_n, dK then dV, B * Hk, Sk, D), which
+  // fa_bwd_seg_sum_kernel adds in segment order.  1: none.
+  int seg_n;
+  float *seg_part;
   // dQ kernel: when non-NULL, workgroup 0 zeroes cnt_zero[0 .. n_cnt_zero)
   // (the split counters of the dK/dV launch that follows on the stream)
   unsigned *cnt_zero;
@@ -540,12 +547,16 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   // split, ranks 2kt and 2kt + 1 are the two halves of block kt < split_kt,
   // then the unsplit blocks follow, heaviest first.
   const int nsplit = (T::KEY_SPLIT && CAUSAL) ? a.split_kt : 0;
+  // Sweep segments (BwdArgs::seg_n): ranks seg_n * kt + 0 .. seg_n - 1 are
+  // the segments of block kt, heaviest block first.
+  const int nseg = a.seg_n;
   const bool split = rank < 2 * nsplit;
-  const int seg = split ? (rank & 1) : 0;
-  const int kt = split ? (rank >> 1)
-                       : (nsplit > 0 ? rank - nsplit
-                                     : ((CAUSAL && a.zigzag) ? zigzag_rank(rank, a.n_blocks)
-                                                             : rank));
+  const int seg = nseg > 1 ? rank % nseg : (split ? (rank & 1) : 0);
+  const int kt = nseg > 1 ? rank / nseg
+                 : split  ? (rank >> 1)
+                          : (nsplit > 0 ? rank - nsplit
+                                        : ((CAUSAL && a.zigzag) ? zigzag_rank(rank, a.n_blocks)
+                                                                : rank));
   const int b = bhk / a.Hk, hk = bhk % a.Hk;
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int kg = w / T::NQH;
@@ -644,11 +655,12 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   const int m_first = CAUSAL ? max(0, k0 - off) : 0;
   const int m_begin = (m_first / BQ) * BQ;
   const int nt_h = (Sq > m_begin) ? (Sq - m_begin + BQ - 1) / BQ : 0;
-  // A split block's segment 0 takes the first half of these tiles,
-  // segment 1 the rest.
+  // Segment seg of a block swept by several workgroups (two for a split
+  // block) takes tiles [n_all * seg / parts, n_all * (seg + 1) / parts).
   const int n_all = nt_h * a.grp;
-  const int t_begin = seg ? n_all / 2 : 0;
-  const int n_tiles = split ? (seg ? n_all - n_all / 2 : n_all / 2) : n_all;
+  const int parts = nseg > 1 ? nseg : (split ? 2 : 1);
+  const int t_begin = (int)((int64_t)n_all * seg / parts);
+  const int n_tiles = (int)((int64_t)n_all * (seg + 1) / parts) - t_begin;
 
   // Per-query rows staged beside each tile, laid out as MFMA accumulator
   // seeds: s_lse = -LSE * log2(e) / cr (-inf past S, so P = 0 there) and
@@ -1113,9 +1125,43 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
     dk_mul = a.sm_scale;
   }
   if (key < Sk) {
+    if (nseg > 1) {
+      float *p = a.seg_part + (((int64_t)seg * 2 * BHk + bhk) * Sk + key) * D;
+      store_row_f32<D>(p, dk, dk_mul, g);
+      store_row_f32<D>(p + (int64_t)BHk * Sk * D, dv, 1.0f, g);
+      return;
+    }
     store_row<E, D>(a.dk + b * a.dk_sb + hk * a.dk_sh + (int64_t)key * a.dk_ss, dk, dk_mul, g);
     store_row<E, D>(a.dv + b * a.dv_sb + hk * a.dv_sh + (int64_t)key * a.dv_ss, dv, 1.0f, g);
   }
+}
+
+// dK and dV of blocks swept in segments: the segments' fp32 rows summed in
+// segment order (reproducible) and converted.  HBM-bound: reads
+// 2 seg_n B Hk Sk D fp32, writes the 16-bit rows; four columns a thread,
+// blockIdx.y picks dK or dV.
+template <typename E, int D>
+__global__ __launch_bounds__(256) void fa_bwd_seg_sum_kernel(BwdArgs a) {
+  const int64_t rows = (int64_t)a.B * a.Hk * a.Sk;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= rows * (D / 4)) return;
+  const int64_t row = i / (D / 4);
+  const int c = 4 * (int)(i % (D / 4));
+  const float *p = a.seg_part + (int64_t)blockIdx.y * rows * D + row * D + c;
+  floatx4 acc = *(const floatx4 *)p;
+#pragma unroll 4
+  for (int s = 1; s < a.seg_n; ++s) {
+    const floatx4 x = *(const floatx4 *)(p + s * 2 * rows * D);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] += x[j];
+  }
+  const int64_t bhk = row / a.Sk, key = row % a.Sk, b = bhk / a.Hk, hk = bhk % a.Hk;
+  f16 *dst = blockIdx.y == 0 ? a.dk + b * a.dk_sb + hk * a.dk_sh + key * a.dk_ss
+                             : a.dv + b * a.dv_sb + hk * a.dv_sh + key * a.dv_ss;
+  vec4<E> v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = (E)acc[j];
+  *(vec4<E> *)(dst + c) = v;
 }
 
 template <typename E, int D, bool CAUSAL, int SPLIT>

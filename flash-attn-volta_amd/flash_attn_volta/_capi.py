@@ -52,6 +52,7 @@ EXPORTED_SYMBOLS = (
     "fa_bwd_rowmax_bytes",
     "fa_bwd_workspace_bytes",
     "fa_bwd_gqa_workspace_bytes",
+    "fa_bwd_best_workspace_bytes",
     "fa_bwd",
     "fa_bwd_gqa",
     "fa_bwd_gqa_noalloc",
@@ -118,6 +119,8 @@ def _declare(lib):
     lib.fa_bwd_workspace_bytes.argtypes = [_ci, _ci, _ci, _ci]
     lib.fa_bwd_gqa_workspace_bytes.restype = ctypes.c_size_t
     lib.fa_bwd_gqa_workspace_bytes.argtypes = [_ci, _ci, _ci, _ci, _ci, _ci, _ci]
+    lib.fa_bwd_best_workspace_bytes.restype = ctypes.c_size_t
+    lib.fa_bwd_best_workspace_bytes.argtypes = [_ci, _ci, _ci, _ci, _ci, _ci, _ci]
     lib.fa_bwd.restype = _ci
     lib.fa_bwd.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp,
                            _vp, _vp, _vp,

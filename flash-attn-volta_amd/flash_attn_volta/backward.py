@@ -134,7 +134,7 @@ class _BwdPlan:
         # (bytes, the same as a C size_t argument)
         n = int(lib.fa_bwd_workspace_bytes(B, Sq, H, D))
         self.ws_plain = (n, ctypes.c_size_t(n))
-        n = int(lib.fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, c))
+        n = int(lib.fa_bwd_best_workspace_bytes(B, Sq, Sk, H, Hk, D, c))
         self.ws_split = (n, ctypes.c_size_t(n))
         if gqa:
             self.name = "fa_bwd_gqa"
@@ -188,7 +188,7 @@ def _backward(do, q, k, v, o, lse, causal, sm_scale, gqa):
 
 
 # The backward's workspace: with split_workspace (the default) it asks for
-# fa_bwd_gqa_workspace_bytes, with which small causal D = 64 / 128 grids run
+# fa_bwd_best_workspace_bytes, with which small causal D = 64 / 128 grids run
 # their split schedule (longest key / query blocks swept by two workgroups;
 # 8-20 % faster on those grids, at up to 80 MiB of fp32 partials); set it
 # to False to cap the workspace at delta's B * H * Sq * 4 bytes (the
@@ -221,13 +221,13 @@ def _run_bwd(do, q, k, v, o, lse, causal, sm_scale, gqa):
           kernel_strides(o), sq_, sk_, sk_)
     with _on_device(q.device):
         # the size that lets small causal D = 64 / 128 grids split their
-        # longest key / query blocks (fa_bwd_gqa_workspace_bytes); delta
+        # longest key / query blocks (fa_bwd_best_workspace_bytes); delta
         # alone otherwise
         key = (B, N, Sk, H, Hk, D, bool(causal), split_workspace)
         ws_bytes = _WS_BYTES.get(key)
         if ws_bytes is None:
             if split_workspace:
-                ws_bytes = lib.fa_bwd_gqa_workspace_bytes(B, N, Sk, H, Hk, D, int(bool(causal)))
+                ws_bytes = lib.fa_bwd_best_workspace_bytes(B, N, Sk, H, Hk, D, int(bool(causal)))
             else:
                 ws_bytes = lib.fa_bwd_workspace_bytes(B, N, H, D)
             _WS_BYTES[key] = ws_bytes

@@ -279,7 +279,7 @@ class _FwdPlan:
         for arr in (*self.st, dq_st, dk_st):
             ints += list(arr)
         ints += [self.ws_bytes,
-                 int(lib.fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, int(self.causal))),
+                 int(lib.fa_bwd_best_workspace_bytes(B, Sq, Sk, H, Hk, D, int(self.causal))),
                  int(lib.fa_bwd_workspace_bytes(B, Sq, H, D))]
         self.cpp = ext.make_plan(ints, self.sm_scale)
         return self.cpp

@@ -232,6 +232,18 @@ size_t fa_bwd_workspace_bytes(int B, int S, int H, int D);
 size_t fa_bwd_gqa_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, int causal);
 
 /*
+ * fa_bwd_gqa_workspace_bytes, or, where the key blocks are fewer than the
+ * workgroups the GPU holds and their sweeps are long (few key/value heads,
+ * whose sweep covers every query head of the group), the larger size with
+ * which fa_bwd / fa_bwd_gqa sweep every key block in segments, one
+ * workgroup each: the fa_bwd_workspace_bytes minimum plus the segments'
+ * fp32 dK and dV rows, which a last launch adds in segment order (0 on bad
+ * sizes).  Results differ from the other schedules' in rounding only and are
+ * bit-reproducible.
+ */
+size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, int causal);
+
+/*
  * Backward attention: (dq, dk, dv) of L = <o, dout> with o = fa_fwd(q,k,v),
  * given the forward's `lse`. Two launches. Causal with D = 32 or 64, and
  * causal D = 128 on grids of at most four workgroups of eight waves per
