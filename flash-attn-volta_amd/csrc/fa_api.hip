@@ -194,21 +194,72 @@ int device_cus() {
   return n;
 }
 
-// Split each tile's rows across two waves when the grid of 128-row
-// workgroups would leave the GPU under-filled: fewer than one round of the
-// resident workgroup slots (`per_cu` per CU), two rounds for causal, whose
-// light blocks finish early and leave the heavy blocks' long sweeps as the
-// critical path.  Used by the forward and both backward kernels (the split
-// is over keys in the forward and dQ, over queries in dK/dV); `rows` is
-// the length of the blocked dimension, `heads` the number of (b, head)
-// pairs the grid covers.  per_cu = 2 for the kernels that run two
-// workgroups per CU; 1 for D = 128 dK/dV, whose registers allow one
-// (measured: unsplit is 11 % faster at (1,4096,8,128) non-causal and 4 %
-// at (1,4096,16,128) causal, split stays 19 % faster at (1,4096,8,128)
-// causal).
-bool row_split(int rows, int64_t heads, bool causal, int per_cu = 2) {
-  const int64_t wgs = (int64_t)((rows + 127) / 128) * heads;
-  return wgs < (int64_t)(causal ? 2 : 1) * per_cu * device_cus();
+// Layouts by grid size.  A layout that splits each tile's rows across two
+// waves (64 output rows a workgroup: twice the waves, half the work each)
+// pays where the grid of 128-row workgroups leaves the GPU under-filled or
+// ends on a nearly empty round; it costs about 15 % on full rounds.  The
+// lines below are in 128-row workgroups (n), two of which make a CU's round;
+// each was measured on both sides (us, same box; 64-row / 128-row layout
+// unless said otherwise).
+int64_t grid128(int rows, int64_t heads) { return (int64_t)((rows + 127) / 128) * heads; }
+
+// Forward, key split in two halves.
+//   causal, D = 64: below 2.5 CUs' worth, and up to 4 on sweeps under 16
+//     tiles of 128 rows ((1,4096,20) 58 / 57, (1,4096,24) 67 / 61,
+//     (2,2048,25) 43 / 40, (1,4096,18) 53 / 55, (8,1024,12) 25 / 28,
+//     (5,1536,12) 32 / 37);
+//   causal, D = 128: below 2, and to 2.25 past 2048 rows ((1,3000,16) 47 / 56,
+//     (1,4096,16) 80 / 82, (1,2048,32) 49 / 45, (2,1024,32) 35 / 28, (1,4096,18)
+//     100 / 97, (1,4096,24) 125 / 112);
+//   not causal: D = 64 up to 2.5 ((1,4096,18) 94 / 103, (1,4096,20) 101 / 105,
+//     (1,4096,22) 119 / 108), D = 128 below one ((1,3800,8) 67 / 67, one
+//     round and more: launch_fwd).
+bool fwd_split2(int D, bool causal, int Sq, int64_t heads) {
+  const int64_t n = grid128(Sq, heads), cus = device_cus();
+  if (causal) {
+    if (D == 64) return n < 4 * cus && (2 * n < 5 * cus || Sq < 2048);
+    if (D == 128) return n < 2 * cus || (4 * n < 9 * cus && Sq > 2048);
+    return n < 4 * cus;
+  }
+  return D == 64 ? 2 * n <= 5 * cus : (D == 128 ? n < cus : n < 2 * cus);
+}
+
+// dQ, key split in two halves.
+//   causal: D = 64 below 2.25, D = 128 below 2.5 (the backward: D = 64
+//     (1,4096,16) 143 / 151, (1,4096,18) 163 / 159 with the dK/dV blocks
+//     unsplit too, (8,1024,12) 78 / 65, (16,512,12) 59 / 50; D = 128
+//     (1,4096,16) 265 / 297, (1,4096,18) 311 / 320, (1,3000,32) 306 / 296);
+//   not causal: D = 64 below two ((1,4096,18) 345 / 325, (1,4096,24) 387 /
+//     374), D = 128 below one ((1,4608,8) 406 / 399, (16,197,12) 61 / 55).
+bool dq_split2(int D, bool causal, int Sq, int64_t heads) {
+  const int64_t n = grid128(Sq, heads), cus = device_cus();
+  if (causal) return D == 64 ? 4 * n < 9 * cus : (D == 128 ? 2 * n < 5 * cus : n < 4 * cus);
+  return n < (D == 128 ? 1 : 2) * cus;
+}
+
+// dK/dV, query split in two halves (the causal D = 128 kernel has one
+// layout).  `heads` counts a sweep segment as a head of its own.
+//   causal: D = 64 below 2.25 (as dq_split2);
+//   not causal: D = 64 below two; D = 128, whose 64-row layout runs one wave
+//     per SIMD, while its grid fits one round ((1,1000,8) 53 / 58, (1,2048,4)
+//     77 / 82, (1,3000,8) 218 / 159).
+bool dkdv_split2(int D, bool causal, int Sk, int64_t heads) {
+  const int64_t n = grid128(Sk, heads), cus = device_cus();
+  if (causal) return D == 64 ? 4 * n < 9 * cus : n < 4 * cus;
+  return D == 128 ? 2 * n <= cus : n < 2 * cus;
+}
+
+// Not causal, D = 64: eight waves, 256 rows a workgroup, one workgroup per CU
+// and round, half the tile DMAs per row.  Pays (1-3 %) on full or nearly full
+// rounds of long sweeps whose rows it does not pad further; elsewhere the
+// 128-row layout's finer rounds win (forward, eight waves / four: (1,4096,16)
+// 68 / 70, (1,4096,30) 137 / 138, (1,4096,26) 127 / 131, (1,4096,24) 121 / 115,
+// (1,4096,36) 192 / 175, (8,577,16) 28 / 24, (32,197,12) 19 / 16, (64,100,12)
+// 20 / 13).
+bool eight_waves_64(int Sq, int Sk, int64_t heads) {
+  const int64_t n = (int64_t)((Sq + 255) / 256) * heads, cus = device_cus(), rem = n % cus;
+  return n >= cus && (rem == 0 || 5 * rem >= 3 * cus) && Sk >= 1024 &&
+         15 * 2 * n <= 16 * grid128(Sq, heads);
 }
 
 // Workgroups of `Kernel` (launched with `threads` per workgroup) resident
@@ -268,54 +319,43 @@ int launch_fwd_split(const fa::FwdArgs &args, hipStream_t stream) {
   return launch_status();
 }
 
-template <typename E, int D, bool CAUSAL, int KSPLIT>
+// launch_fwd_split in the pre-scaled mode where it applies.  (Not in the
+// unsplit D = 128 layout: the -max seed's 16 registers would push it past
+// 256 VGPRs, measured +3-4 % on the grids that use it.)
+template <typename E, int D, bool CAUSAL, int KSPLIT, int NW = 4>
 int launch_fwd_mode(const fa::FwdArgs &a, hipStream_t stream) {
-  // Non-causal D = 64 grids of at least one 256-query tile per CU: eight
-  // waves, 256 queries per workgroup sharing each K / V tile (half the
-  // tile DMAs per query).
-  if constexpr (D == 64 && !CAUSAL && KSPLIT == 1) {
-    if ((int64_t)((a.Sq + 255) / 256) * a.B * a.H >= device_cus()) {
-      if constexpr (std::is_same<E, fa::f16>::value) {
-        if (fwd_prescaled<E>(a)) return launch_fwd_split<E, D, CAUSAL, 1, true, 8>(a, stream);
-      }
-      return launch_fwd_split<E, D, CAUSAL, 1, false, 8>(a, stream);
-    }
-  }
-  // Non-causal D = 128 key-split grids of at least one 128-query tile per
-  // CU: eight waves (four query groups x two key halves) sharing each K / V
-  // tile.
-  if constexpr (D == 128 && !CAUSAL && KSPLIT == 2) {
-    if ((int64_t)((a.Sq + 127) / 128) * a.B * a.H >= device_cus()) {
-      if constexpr (std::is_same<E, fa::f16>::value) {
-        if (fwd_prescaled<E>(a)) return launch_fwd_split<E, D, CAUSAL, 2, true, 8>(a, stream);
-      }
-      return launch_fwd_split<E, D, CAUSAL, 2, false, 8>(a, stream);
-    }
-  }
-  // (not the unsplit D = 128 layout: the -max seed's 16 registers would
-  // push it past 256 VGPRs, measured +3-4 % on the grids that use it)
   if constexpr (std::is_same<E, fa::f16>::value && !(D == 128 && KSPLIT == 1)) {
-    if (fwd_prescaled<E>(a)) return launch_fwd_split<E, D, CAUSAL, KSPLIT, true>(a, stream);
+    if (fwd_prescaled<E>(a)) return launch_fwd_split<E, D, CAUSAL, KSPLIT, true, NW>(a, stream);
   }
-  return launch_fwd_split<E, D, CAUSAL, KSPLIT, false>(a, stream);
+  return launch_fwd_split<E, D, CAUSAL, KSPLIT, false, NW>(a, stream);
 }
 
 template <typename E, int D, bool CAUSAL>
 int launch_fwd(const fa::FwdArgs &a, hipStream_t stream) {
-  // Non-causal grids of at most one 64-query workgroup per CU, where the
-  // four-wave key-split layout would run one wave per SIMD: eight waves per
-  // workgroup, each query group's keys in four parts of 128-key tiles --
-  // twice the waves in flight on the same grid.
+  const int64_t heads = (int64_t)a.B * a.H;
   if constexpr (!CAUSAL && D >= 64) {
-    if ((int64_t)((a.Sq + 63) / 64) * a.B * a.H <= device_cus()) {
-      if constexpr (std::is_same<E, fa::f16>::value) {
-        if (fwd_prescaled<E>(a)) return launch_fwd_split<E, D, CAUSAL, 4, true, 8>(a, stream);
-      }
-      return launch_fwd_split<E, D, CAUSAL, 4, false, 8>(a, stream);
-    }
+    // Grids of at most one 64-query workgroup per CU, where the four-wave
+    // key-split layout would run one wave per SIMD: eight waves per
+    // workgroup, each query group's keys in four parts of 128-key tiles --
+    // twice the waves in flight on the same grid.  At D = 128 from 16 key
+    // tiles on (its merge and larger tiles cost more below: (2,300,8) 11.4 us,
+    // 9.4 in the two-part layout, (1,512,4) 11.8 / 10.7, (1,1000,8) 15.6 /
+    // 15.1, (2,1024,4) 15.9 / 15.9, (1,2048,4) 23.0 / 25.4; D = 64 (4,256,12)
+    // 7.5 / 8.2, (1,1000,12) 10.8 / 11.7).
+    if ((int64_t)((a.Sq + 63) / 64) * heads <= device_cus() && (D == 64 || a.Sk >= 1024))
+      return launch_fwd_mode<E, D, CAUSAL, 4, 8>(a, stream);
   }
-  return row_split(a.Sq, (int64_t)a.B * a.H, CAUSAL) ? launch_fwd_mode<E, D, CAUSAL, 2>(a, stream)
-                                                     : launch_fwd_mode<E, D, CAUSAL, 1>(a, stream);
+  if constexpr (!CAUSAL && D == 64) {
+    if (eight_waves_64(a.Sq, a.Sk, heads)) return launch_fwd_mode<E, D, CAUSAL, 1, 8>(a, stream);
+  }
+  if constexpr (!CAUSAL && D == 128) {
+    // exactly one round of eight-wave key-split workgroups (128 queries
+    // each), long sweeps: (1,4096,8) 69 us, 72 unsplit; (1,4608,8) 131 / 109
+    if (grid128(a.Sq, heads) == device_cus() && a.Sk >= 2048)
+      return launch_fwd_mode<E, D, CAUSAL, 2, 8>(a, stream);
+  }
+  return fwd_split2(D, CAUSAL, a.Sq, heads) ? launch_fwd_mode<E, D, CAUSAL, 2>(a, stream)
+                                            : launch_fwd_mode<E, D, CAUSAL, 1>(a, stream);
 }
 
 template <typename E, int D>
@@ -391,19 +431,23 @@ int launch_dkdv(const fa::BwdArgs &a, hipStream_t stream) {
   if constexpr (D == 64 && CAUSAL) {
     if (a.split_kt > 0) return launch_dkdv_split<E, D, CAUSAL, 2>(a, stream);
   }
-  return row_split(a.Sk, (int64_t)a.B * a.Hk * a.seg_n, CAUSAL, D >= 128 ? 1 : 2)
+  return dkdv_split2(D, CAUSAL, a.Sk, (int64_t)a.B * a.Hk * a.seg_n)
              ? launch_dkdv_split<E, D, CAUSAL, 2>(a, stream)
              : launch_dkdv_split<E, D, CAUSAL, 1>(a, stream);
 }
 
 template <typename E, int D, bool CAUSAL>
 int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
-  const bool split = row_split(a.Sq, (int64_t)a.B * a.H, CAUSAL);
-  // Non-causal grids of at least one eight-wave workgroup per CU: eight
-  // waves sharing each K / V tile, as in the forward (D = 64: 256 queries,
-  // no key split; D = 128 where the key split is chosen: 128 queries)
+  const int64_t heads = (int64_t)a.B * a.H;
+  const bool split = dq_split2(D, CAUSAL, a.Sq, heads);
+  // Eight waves sharing each K / V tile, as in the forward: D = 64 (256
+  // queries, no key split) below two rounds ((1,4096,16) 235.7 us the
+  // backward, 238.2 with four waves, (1,4096,30) 466 / 494, (1,4096,32) 466 /
+  // 462, (4,4096,16) 947 / 924), D = 128 (128 queries, key split) on exactly
+  // one round ((1,4096,8) 234 / 239, (1,4096,14) 442 / 425).
   if constexpr (!CAUSAL && D == 64) {
-    if (!split && (int64_t)((a.Sq + 255) / 256) * a.B * a.H >= device_cus()) {
+    if (!split && eight_waves_64(a.Sq, a.Sk, heads) &&
+        (int64_t)((a.Sq + 255) / 256) * heads < 2 * (int64_t)device_cus()) {
       if constexpr (std::is_same<E, fa::f16>::value) {
         if (a.c <= 1.0f) return launch_dq_split<E, D, CAUSAL, 1, true, 8>(a, stream);
       }
@@ -411,7 +455,7 @@ int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
     }
   }
   if constexpr (!CAUSAL && D == 128) {
-    if (split && (int64_t)((a.Sq + 127) / 128) * a.B * a.H >= device_cus()) {
+    if (grid128(a.Sq, heads) == device_cus() && a.Sk >= 2048) {
       if constexpr (std::is_same<E, fa::f16>::value) {
         if (a.c <= 1.0f) return launch_dq_split<E, D, CAUSAL, 2, true, 8>(a, stream);
       }
@@ -784,7 +828,7 @@ struct BalPlan {
 
 BalPlan bal_plan(const Shape &s, int causal) {
   if (!causal || s.Sq != s.Sk) return BalPlan{0};
-  if (!row_split(s.Sq, (int64_t)s.B * s.H, true)) return BalPlan{0};
+  if (!fwd_split2(s.D, true, s.Sq, (int64_t)s.B * s.H)) return BalPlan{0};
   const int nb = (s.Sq + 63) / 64;
   const int64_t grid = (int64_t)nb * s.B * s.H;
   if (nb < kBalMinTiles) return BalPlan{0};
@@ -1032,7 +1076,7 @@ DkdvSplit dkdv_split_plan(const Shape &s, int causal) {
     if (causal_tiles(s, 0, T::BK, T::BQ) < 64 && 2 * blocks > device_cus()) return DkdvSplit{};
     return split_plan_for<T>(s, [](int64_t t0) { return t0 / 16 > 4 ? t0 / 16 : (int64_t)4; });
   }
-  if (s.D == 64 && row_split(s.Sk, (int64_t)s.B * s.Hk, true, 2))
+  if (s.D == 64 && dkdv_split2(64, true, s.Sk, (int64_t)s.B * s.Hk))
     return split_plan_for<fa::DkdvTile<64, 2>>(s, [](int64_t t0) { return t0 / 3; });
   return DkdvSplit{};
 }
@@ -1057,7 +1101,7 @@ DqSplit dq_split_plan(const Shape &s, int causal) {
   DqSplit p;
   if (!causal || (s.D != 64 && s.D != 128)) return p;
   const int64_t bh = (int64_t)s.B * s.H;
-  const bool sp = row_split(s.Sq, bh, true);
+  const bool sp = dq_split2(s.D, true, s.Sq, bh);
   const int BM = s.D == 64 ? (sp ? fa::DqTile<64, 2>::BM : fa::DqTile<64, 1>::BM)
                            : (sp ? fa::DqTile<128, 2>::BM : fa::DqTile<128, 1>::BM);
   constexpr int BN = fa::DqTile<64, 1>::BN;
@@ -1400,8 +1444,8 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
     f.with_pre = true;
     f.akv.seg_n = seg_n;
     f.akv.seg_part = seg_part;
-    f.kv_split2 = plan.split_kt > 0 || row_split(s.Sk, (int64_t)s.B * s.Hk * seg_n, true, 2);
-    f.q_split2 = row_split(s.Sq, (int64_t)s.B * s.H, true);
+    f.kv_split2 = plan.split_kt > 0 || dkdv_split2(s.D, true, s.Sk, (int64_t)s.B * s.Hk * seg_n);
+    f.q_split2 = dq_split2(s.D, true, s.Sq, (int64_t)s.B * s.H);
     hipStream_t st = static_cast<hipStream_t>(stream);
     FA_DISPATCH(launch_bwd_fused, s, causal, f, st);
   }
@@ -1450,8 +1494,8 @@ int run_bwd_blocks(const void *dout, const void *q, const void *k, const void *v
                     nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, &f.aq)))
     return rc;
   f.with_pre = false;
-  f.kv_split2 = row_split(s.Sk, (int64_t)s.B * s.Hk, true, 2);
-  f.q_split2 = row_split(s.Sq, (int64_t)s.B * s.H, true);
+  f.kv_split2 = dkdv_split2(s.D, true, s.Sk, (int64_t)s.B * s.Hk);
+  f.q_split2 = dq_split2(s.D, true, s.Sq, (int64_t)s.B * s.H);
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_bwd_fused, s, causal, f, st);
 }

@@ -655,12 +655,16 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   const int m_first = CAUSAL ? max(0, k0 - off) : 0;
   const int m_begin = (m_first / BQ) * BQ;
   const int nt_h = (Sq > m_begin) ? (Sq - m_begin + BQ - 1) / BQ : 0;
-  // Segment seg of a block swept by several workgroups (two for a split
-  // block) takes tiles [n_all * seg / parts, n_all * (seg + 1) / parts).
+  // A block swept by several workgroups (two for a split block): equal runs
+  // of tiles, the last n_all % parts segments one tile longer.
   const int n_all = nt_h * a.grp;
-  const int parts = nseg > 1 ? nseg : (split ? 2 : 1);
-  const int t_begin = (int)((int64_t)n_all * seg / parts);
-  const int n_tiles = (int)((int64_t)n_all * (seg + 1) / parts) - t_begin;
+  int t_begin = 0, n_tiles = n_all;
+  if (nseg > 1 || split) {
+    const int parts = nseg > 1 ? nseg : 2;
+    const int base = n_all / parts, longer = parts - n_all % parts;   // first longer segment
+    t_begin = base * seg + max(0, seg - longer);
+    n_tiles = base + (seg >= longer ? 1 : 0);
+  }
 
   // Per-query rows staged beside each tile, laid out as MFMA accumulator
   // seeds: s_lse = -LSE * log2(e) / cr (-inf past S, so P = 0 there) and
