@@ -57,6 +57,17 @@ def _table_strides(t: torch.Tensor):
                                 0 if t.size(1) == 1 else int(t.stride(1)))
 
 
+def _tables(cos, sin, B: int, S: int, D: int, dtype, device):
+    """cos and sin as _table gives them, of one shape and, since the kernels
+    read both by cos's strides, of equal strides."""
+    cos = _table(cos, "cos", B, S, D, dtype, device)
+    sin = _table(sin, "sin", B, S, D, dtype, device)
+    _require(cos.shape[0] == sin.shape[0], "cos and sin must have the same shape")
+    if list(_table_strides(cos)) != list(_table_strides(sin)):
+        cos, sin = cos.contiguous(), sin.contiguous()
+    return cos, sin
+
+
 def _weight(w, name: str, D: int, dtype, device):
     if w is None:
         return None
@@ -92,9 +103,7 @@ def rope_qk_forward(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: to
     _check_qk(q, k)
     B, S, H, D = q.shape
     Hk = k.shape[2]
-    cos = _table(cos, "cos", B, S, D, q.dtype, q.device)
-    sin = _table(sin, "sin", B, S, D, q.dtype, q.device)
-    _require(cos.shape[0] == sin.shape[0], "cos and sin must have the same shape")
+    cos, sin = _tables(cos, sin, B, S, D, q.dtype, q.device)
     wq = _weight(q_norm_weight, "q_norm_weight", D, q.dtype, q.device)
     wk = _weight(k_norm_weight, "k_norm_weight", D, q.dtype, q.device)
     q_out = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
@@ -138,8 +147,7 @@ def rope_qk_backward(dq_out: torch.Tensor, dk_out: torch.Tensor, q: torch.Tensor
         dq_out = dq_out.to(q.dtype)
     if dk_out.dtype != q.dtype:
         dk_out = dk_out.to(q.dtype)
-    cos = _table(cos, "cos", B, S, D, q.dtype, q.device)
-    sin = _table(sin, "sin", B, S, D, q.dtype, q.device)
+    cos, sin = _tables(cos, sin, B, S, D, q.dtype, q.device)
     wq = _weight(q_norm_weight, "q_norm_weight", D, q.dtype, q.device)
     wk = _weight(k_norm_weight, "k_norm_weight", D, q.dtype, q.device)
     dq = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
