@@ -1,5 +1,6 @@
-// Autograd node of flash_attn / flash_attn_gqa in C++ (Python module
-// flash_attn_volta._fa_torch), a client of the C ABI in fa_mi355x.h.
+// Autograd nodes of flash_attn / flash_attn_gqa and apply_rotary_qk in C++
+// (Python module flash_attn_volta._fa_torch), a client of the C ABI in
+// fa_mi355x.h.
 //
 // The reference's autograd.Function (flash_attn_volta/autograd.py:19-59)
 // is Python, and so is this package's (autograd.py).  A Python backward
@@ -16,16 +17,26 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <optional>
+#include <tuple>
 #include <unordered_set>
 #include <vector>
 
 #include "fa_mi355x.h"
+
+// Weak, so that the module still loads beside a library of another ABI
+// version without them, as far as the version check below.
+extern "C" {
+__attribute__((weak)) decltype(fa_rope_qk_fwd) fa_rope_qk_fwd;
+__attribute__((weak)) decltype(fa_rope_qk_bwd) fa_rope_qk_bwd;
+__attribute__((weak)) decltype(fa_rope_qk_workspace_bytes) fa_rope_qk_workspace_bytes;
+}
 
 namespace {
 
@@ -190,6 +201,136 @@ std::optional<Tensor> attn(int64_t handle, const Tensor &q, const Tensor &k, con
   return FlashAttnFn::apply(q, k, v, handle, split);
 }
 
+// The QK-norm + rotary prologue (rope.py's apply_rotary_qk) on tensors the
+// kernels read in place.  A step of it is three kernels of some 45 us at
+// (1, 4096, 32 / 8 heads, 128); a Python node around them took 178 us of host
+// time a step.
+using OptTensor = std::optional<Tensor>;
+
+int dtype_of(const Tensor &t) {
+  return t.scalar_type() == at::kHalf ? FA_DTYPE_F16 : FA_DTYPE_BF16;
+}
+
+const void *ptr_or_null(const OptTensor &t) { return t && t->defined() ? t->data_ptr() : nullptr; }
+
+// (b, s) strides of a (1 or B, S, D) or (S, D) table, 0 for size-1 dims.
+void table_strides(const Tensor &t, int64_t (&st)[2]) {
+  const int64_t d = t.dim();
+  st[0] = d == 2 || t.size(0) == 1 ? 0 : t.stride(0);
+  st[1] = t.size(d - 2) == 1 ? 0 : t.stride(d - 2);
+}
+
+struct RopeFn : public torch::autograd::Function<RopeFn> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k,
+                               const Tensor &cos, const Tensor &sin, const OptTensor &wq,
+                               const OptTensor &wk, double eps) {
+    const c10::DeviceGuard guard(q.device());
+    Tensor qo = at::empty(q.sizes(), q.options()), ko = at::empty(k.sizes(), k.options());
+    int64_t q_st[4], k_st[4], qo_st[4], ko_st[4], cs[2];
+    kernel_strides(q, q_st);
+    kernel_strides(k, k_st);
+    kernel_strides(qo, qo_st);
+    kernel_strides(ko, ko_st);
+    table_strides(cos, cs);
+    check(fa_rope_qk_fwd(q.data_ptr(), k.data_ptr(), qo.data_ptr(), ko.data_ptr(), cos.data_ptr(),
+                         sin.data_ptr(), ptr_or_null(wq), ptr_or_null(wk), (float)eps,
+                         (int)q.size(0), (int)q.size(1), (int)q.size(2), (int)k.size(2),
+                         (int)q.size(3), q_st, k_st, qo_st, ko_st, cs, dtype_of(q), stream_of(q)),
+          "fa_rope_qk_fwd");
+    // the forward's inputs are needed again only to recompute a norm
+    ctx->save_for_backward({wq ? q : Tensor(), wk ? k : Tensor(), cos, sin, wq.value_or(Tensor()),
+                            wk.value_or(Tensor())});
+    ctx->saved_data["eps"] = eps;
+    return {qo, ko};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const Tensor &cos = s[2], &sin = s[3], &wq = s[4], &wk = s[5];
+    const double eps = ctx->saved_data["eps"].toDouble();
+    const c10::DeviceGuard guard(cos.device());
+    const auto opt = cos.options();
+    int64_t g_st[2][4], x_st[2][4], d_st[2][4], cs[2];
+    Tensor g[2], x[2], d[2], dw[2];
+    for (int i = 0; i < 2; ++i) {
+      g[i] = grads[i].scalar_type() == cos.scalar_type() ? grads[i]
+                                                         : grads[i].to(cos.scalar_type());
+      if (!kernel_strides(g[i], g_st[i]) || !aligned(g[i])) {
+        g[i] = g[i].clone(at::MemoryFormat::Contiguous);
+        kernel_strides(g[i], g_st[i]);
+      }
+      x[i] = s[i].defined() ? s[i] : g[i];   // read for a normed side only
+      kernel_strides(x[i], x_st[i]);
+      d[i] = at::empty(g[i].sizes(), opt);
+      kernel_strides(d[i], d_st[i]);
+      if (s[4 + i].defined()) dw[i] = at::empty({g[i].size(3)}, opt.dtype(at::kFloat));
+    }
+    table_strides(cos, cs);
+    const int B = (int)g[0].size(0), S = (int)g[0].size(1), H = (int)g[0].size(2),
+              Hk = (int)g[1].size(2), D = (int)g[0].size(3);
+    Tensor ws;
+    if (wq.defined() || wk.defined())
+      ws = at::empty({(int64_t)fa_rope_qk_workspace_bytes(B, S, H, Hk, D)}, opt.dtype(at::kByte));
+    auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
+    check(fa_rope_qk_bwd(g[0].data_ptr(), g[1].data_ptr(), x[0].data_ptr(), x[1].data_ptr(),
+                         cos.data_ptr(), sin.data_ptr(), ptr(wq), ptr(wk), (float)eps,
+                         d[0].data_ptr(), d[1].data_ptr(), static_cast<float *>(ptr(dw[0])),
+                         static_cast<float *>(ptr(dw[1])), ptr(ws),
+                         ws.defined() ? (size_t)ws.numel() : 0, B, S, H, Hk, D, g_st[0], g_st[1],
+                         x_st[0], x_st[1], d_st[0], d_st[1], cs, dtype_of(cos), stream_of(cos)),
+          "fa_rope_qk_bwd");
+    for (int i = 0; i < 2; ++i)
+      if (dw[i].defined()) dw[i] = dw[i].to(s[4 + i].scalar_type());
+    return {d[0], d[1], Tensor(), Tensor(), dw[0], dw[1], Tensor()};
+  }
+};
+
+// (q_out, k_out) with the node recorded, or None for anything the kernels do
+// not take in place as it is (other dtypes, devices and layouts, empty or
+// misaligned tensors, tables that need a cast or have unequal strides or
+// gradients, invalid arguments): the caller's general path copies, casts or
+// raises.
+std::optional<std::tuple<Tensor, Tensor>> rope(const Tensor &q, const Tensor &k, const Tensor &cos,
+                                               const Tensor &sin, const OptTensor &wq,
+                                               const OptTensor &wk, double eps) {
+  if (q.dim() != 4 || k.dim() != 4 || !q.is_cuda()) return std::nullopt;
+  const auto dt = q.scalar_type();
+  const int64_t B = q.size(0), S = q.size(1), H = q.size(2), D = q.size(3), Hk = k.size(2);
+  if ((dt != at::kHalf && dt != at::kBFloat16) || q.numel() == 0 || k.numel() == 0 ||
+      (D != 16 && D != 32 && D != 64 && D != 128) || k.size(0) != B || k.size(1) != S ||
+      k.size(3) != D || B > INT32_MAX || S > INT32_MAX ||
+      (double)B * S * (double)std::max(H, Hk) > 2147483647.0)
+    return std::nullopt;
+  auto same = [&](const Tensor &t) {
+    return t.scalar_type() == dt && t.device() == q.device() && aligned(t);
+  };
+  int64_t st[4];
+  if (!same(q) || !same(k) || !kernel_strides(q, st) || !kernel_strides(k, st))
+    return std::nullopt;
+  for (const Tensor *t : {&cos, &sin}) {
+    const int64_t d = t->dim();
+    if ((d != 2 && d != 3) || t->size(d - 1) != D || t->size(d - 2) != S ||
+        (d == 3 && t->size(0) != 1 && t->size(0) != B) || !same(*t) || t->requires_grad() ||
+        t->stride(d - 1) != 1)
+      return std::nullopt;
+    int64_t ts[2];
+    table_strides(*t, ts);
+    if (ts[0] < 0 || ts[1] < 0 || ts[0] % 8 != 0 || ts[1] % 8 != 0) return std::nullopt;
+  }
+  int64_t c_st[2], s_st[2];
+  table_strides(cos, c_st);
+  table_strides(sin, s_st);
+  if (cos.sizes() != sin.sizes() || c_st[0] != s_st[0] || c_st[1] != s_st[1]) return std::nullopt;
+  for (const OptTensor *w : {&wq, &wk}) {
+    if (!*w) continue;
+    if ((*w)->dim() != 1 || (*w)->size(0) != D || !same(**w) || !(*w)->is_contiguous() ||
+        !(std::isfinite(eps) && eps >= 0.0))
+      return std::nullopt;
+  }
+  variable_list r = RopeFn::apply(q, k, cos, sin, wq, wk, eps);
+  return std::make_tuple(r[0], r[1]);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_fa_torch, m) {
@@ -205,8 +346,9 @@ PYBIND11_MODULE(_fa_torch, m) {
                  (int)FA_ABI_VERSION, (int)fa_abi_version());
     throw pybind11::error_already_set();
   }
-  m.doc() = "C++ autograd node of flash_attn_volta's flash_attn / flash_attn_gqa";
+  m.doc() = "C++ autograd nodes of flash_attn_volta's flash_attn / flash_attn_gqa / apply_rotary_qk";
   m.def("make_plan", &make_plan, "register a launch plan (ints, sm_scale) -> handle");
+  m.def("rope", &rope, "QK-norm + rotary prologue, recording the C++ backward node, or None");
   m.def("attn", &attn, "forward of a plan, recording the C++ backward node");
   m.attr("PLAN_INTS") = (int64_t)kPlanInts;
 }

@@ -28,6 +28,7 @@ import ctypes
 import torch
 
 from . import _capi
+from .autograd import _compiling, _cpp, _transforms_active
 from .forward import (FlashAttnArgumentError, _DTYPES, _kernel_ready, _on_device, _require,
                       _stream_ptr, kernel_strides)
 
@@ -240,4 +241,10 @@ def apply_rotary_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: to
         (q_out, k_out): contiguous (B, S, H, D) / (B, S, Hk, D) in q's dtype,
         ready for flash_attn / flash_attn_gqa.
     """
+    if _cpp is not None and not _transforms_active() and not _compiling() and all(
+            isinstance(t, torch.Tensor) for t in (q, k, cos, sin)) and all(
+            w is None or isinstance(w, torch.Tensor) for w in (q_norm_weight, k_norm_weight)):
+        out = _cpp.rope(q, k, cos, sin, q_norm_weight, k_norm_weight, float(eps))
+        if out is not None:
+            return out
     return _RopeQkFn.apply(q, k, cos, sin, q_norm_weight, k_norm_weight, float(eps))
