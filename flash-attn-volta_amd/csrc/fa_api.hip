@@ -28,13 +28,21 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 struct Shape {
   int B, Sq, Sk, H, Hk, D;
   int dtype;   // FA_DTYPE_F16 or FA_DTYPE_BF16
+  int half_cols;   // FA_HALF_COLS: rows of 16 columns in memory, D = 32
+  int cols() const { return half_cols ? D / 2 : D; }
 };
+
+// The sizes of an entry point that takes FA_HALF_COLS in its dtype.
+Shape shape_of(int B, int Sq, int Sk, int H, int Hk, int D, int dtype) {
+  return Shape{B, Sq, Sk, H, Hk, D, dtype & ~FA_HALF_COLS, (dtype & FA_HALF_COLS) != 0};
+}
 
 int check_shape(const Shape &s) {
   if (s.dtype != FA_DTYPE_F16 && s.dtype != FA_DTYPE_BF16) return FA_ERR_DTYPE;
   if (s.B <= 0 || s.Sq <= 0 || s.Sk <= 0 || s.H <= 0 || s.Hk <= 0) return FA_ERR_SHAPE;
   if (s.H % s.Hk != 0) return FA_ERR_SHAPE;
   if (s.D != 32 && s.D != 64 && s.D != 128) return FA_ERR_HEAD_DIM;
+  if (s.half_cols && s.D != 32) return FA_ERR_HEAD_DIM;
   // Per-(b,h) row offsets use 32-bit query/key indices and the grid is 1-D.
   if (s.Sq > (1 << 30) || s.Sk > (1 << 30)) return FA_ERR_TOO_LARGE;
   const int64_t bh = (int64_t)s.B * s.H;
@@ -96,12 +104,20 @@ int check_tensor(const void *p, const int64_t *st, int B, int S, int H, int D, b
   return FA_OK;
 }
 
+int check_rows(const void *p, const int64_t *st, const Shape &s, int S, int heads, bool output) {
+  const int rc = check_tensor(p, st, s.B, S, heads, s.cols(), output, kMaxTileRows);
+  // rows of 16 columns: a head under 2^31 bytes (fa_common.hpp, past_cols)
+  if (rc == FA_OK && s.half_cols && S > 1 && (double)(S - 1) * st[1] * 2 + 2 * s.D > INT32_MAX)
+    return FA_ERR_TOO_LARGE;
+  return rc;
+}
+
 int check_q_like(const void *p, const int64_t *st, const Shape &s, bool output = false) {
-  return check_tensor(p, st, s.B, s.Sq, s.H, s.D, output, kMaxTileRows);
+  return check_rows(p, st, s, s.Sq, s.H, output);
 }
 
 int check_kv_like(const void *p, const int64_t *st, const Shape &s, bool output = false) {
-  return check_tensor(p, st, s.B, s.Sk, s.Hk, s.D, output, kMaxTileRows);
+  return check_rows(p, st, s, s.Sk, s.Hk, output);
 }
 
 // Kernel view of a tensor with S rows per head; a single row's sequence
@@ -742,6 +758,7 @@ fa::FwdArgs fwd_args(const void *q, const void *k, const void *v, void *o, float
   a.off = s.Sk - s.Sq;
   a.c = kernel_scale(sm_scale);
   a.neg = sm_scale < 0.0f;
+  a.cols = s.cols();
   return a;
 }
 
@@ -791,6 +808,7 @@ int run_fwd_splitkv(const void *q, const void *k, const void *v, void *o, float 
   L.c.Sq = s.Sq;
   L.c.H = s.H;
   L.c.n_splits = plan.n_splits;
+  L.c.cols = s.cols();
   L.n_splits = plan.n_splits;
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_fwd_splitkv, s, causal, L, st);
@@ -933,6 +951,7 @@ int run_fwd_ws(const void *q, const void *k, const void *v, void *o, float *lse,
   L.c.B = s.B;
   L.c.Sq = s.Sq;
   L.c.H = s.H;
+  L.c.cols = s.cols();
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_fwd_bal, s, causal, L, st);
 }
@@ -966,6 +985,7 @@ int run_pre(const void *o, const void *dout, float *delta, float *rmax, const Sh
   a.B = s.B;
   a.S = s.Sq;
   a.H = s.H;
+  a.cols = s.cols();
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool bf = s.dtype == FA_DTYPE_BF16;
   switch (s.D) {
@@ -1007,6 +1027,7 @@ int bwd_common(const void *dout, const void *q, const void *k, const void *v, co
   a.lse_mul = lse_seed_mul(a.c, s.dtype);
   a.sm_scale = sm_scale;
   a.neg = sm_scale < 0.0f;
+  a.cols = s.cols();
   a.seg_n = 1;
   *out = a;
   return FA_OK;
@@ -1439,6 +1460,7 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
     f.pre.B = s.B;
     f.pre.S = s.Sq;
     f.pre.H = s.H;
+    f.pre.cols = s.cols();
     f.pre.cnt_zero = cnt;
     f.pre.n_cnt_zero = (int)plan.slots;
     f.with_pre = true;
@@ -1807,7 +1829,7 @@ int fa_fwd_gqa(const void *q, const void *k, const void *v, void *o, float *lse,
                const int64_t q_strides[4], const int64_t k_strides[4],
                const int64_t v_strides[4], const int64_t o_strides[4],
                float sm_scale, int causal, int dtype, void *stream) {
-  return run_fwd(q, k, v, o, lse, Shape{B, Sq, Sk, H, Hk, D, dtype}, q_strides, k_strides, v_strides,
+  return run_fwd(q, k, v, o, lse, shape_of(B, Sq, Sk, H, Hk, D, dtype), q_strides, k_strides, v_strides,
                  o_strides, sm_scale, causal, stream);
 }
 
@@ -1840,7 +1862,8 @@ int fa_fwd_ws(const void *q, const void *k, const void *v, void *o, float *lse,
               const int64_t q_strides[4], const int64_t k_strides[4],
               const int64_t v_strides[4], const int64_t o_strides[4],
               float sm_scale, int causal, int dtype, void *stream) {
-  return run_fwd_ws(q, k, v, o, lse, workspace, workspace_bytes, Shape{B, Sq, Sk, H, Hk, D, dtype},
+  return run_fwd_ws(q, k, v, o, lse, workspace, workspace_bytes,
+                    shape_of(B, Sq, Sk, H, Hk, D, dtype),
                     q_strides, k_strides, v_strides, o_strides, sm_scale, causal, stream);
 }
 
@@ -1904,7 +1927,7 @@ int fa_bwd_gqa(const void *dout, const void *q, const void *k, const void *v,
                const int64_t dk_strides[4], const int64_t dv_strides[4],
                float sm_scale, int causal, int dtype, void *stream) {
   return run_bwd(dout, q, k, v, o, lse, dq, dk, dv, workspace, workspace_bytes,
-                 Shape{B, Sq, Sk, H, Hk, D, dtype}, do_strides, q_strides, k_strides, v_strides,
+                 shape_of(B, Sq, Sk, H, Hk, D, dtype), do_strides, q_strides, k_strides, v_strides,
                  o_strides, dq_strides, dk_strides, dv_strides, sm_scale, causal, stream);
 }
 

@@ -125,6 +125,7 @@ struct BwdArgs {
   float lse_mul;
   float sm_scale;       // signed scale applied to dQ and dK
   int neg;              // 1 when sm_scale < 0 (K or Q negated in S recompute)
+  int cols;             // columns of a row in memory: D, or 16 with D = 32 (past_cols)
   int zigzag;           // causal block order: 1 zigzag heavy / light, 0 heaviest first
   // Causal key-block split (dK/dV layouts with KEY_SPLIT): key blocks
   // [0, split_kt) of every (b, key/value head) are each swept by two
@@ -162,6 +163,7 @@ struct PreArgs {
   float *delta;
   float *rmax;   // row-group maxima (BwdArgs::rmax), (B, H, G, 2); NULL: not written
   int B, S, H;
+  int cols;      // columns of a row in memory (BwdArgs)
   // when non-NULL, workgroup 0 zeroes cnt_zero[0 .. n_cnt_zero) (the
   // key-block split counters of the fused backward launch that follows)
   unsigned *cnt_zero;
@@ -201,8 +203,9 @@ __global__ __launch_bounds__(256) void fa_bwd_preprocess_kernel(PreArgs a) {
     vec8<E> ov[D / 16], gv[D / 16];
 #pragma unroll
     for (int c = 0; c < D / 16; ++c) {
-      ov[c] = ld8<E>(po + 16 * c);
-      gv[c] = ld8<E>(pg + 16 * c);
+      const bool none = past_cols<D>(16 * c, a.cols);
+      ov[c] = none ? vec8<E>{} : ld8<E>(po + 16 * c);
+      gv[c] = none ? vec8<E>{} : ld8<E>(pg + 16 * c);
     }
 #pragma unroll
     for (int c = 0; c < D / 16; ++c)
@@ -264,12 +267,14 @@ struct DsScale {
 // Store a D^T x 32 accumulator set (lane = row `row`, slots = columns) as
 // row `row` of a (.., D) tensor of element type E, scaled by `mul`.
 template <typename E, int D>
-__device__ __forceinline__ void store_row(f16 *dst, const floatx16 (&acc)[D / 32], float mul, int g) {
+__device__ __forceinline__ void store_row(f16 *dst, const floatx16 (&acc)[D / 32], float mul, int g,
+                                          int cols) {
 #pragma unroll
   for (int d = 0; d < D / 32; ++d) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       vec4<E> v4;
+      if (past_cols<D>(c_row(4 * r, g), cols)) continue;
 #pragma unroll
       for (int j = 0; j < 4; ++j) v4[j] = (E)(acc[d][4 * r + j] * mul);
       *(vec4<E> *)(dst + 32 * d + c_row(4 * r, g)) = v4;
@@ -325,10 +330,11 @@ __device__ __forceinline__ void dq_split_combine(const BwdArgs &a, int nt) {
 // Load a lane's D/16 B-operand fragments of row `row` (clamped to S-1).
 template <typename E, int D>
 __device__ __forceinline__ void load_row_frags(vec8<E> (&f)[D / 16], const f16 *head, int64_t ss,
-                                               int row, int S, int g) {
+                                               int row, int S, int g, int cols) {
   const f16 *p = head + (int64_t)min(row, S - 1) * ss + 8 * g;
 #pragma unroll
-  for (int c = 0; c < D / 16; ++c) f[c] = ld8<E>(p + 16 * c);
+  for (int c = 0; c < D / 16; ++c)
+    f[c] = past_cols<D>(16 * c, cols) ? vec8<E>{} : ld8<E>(p + 16 * c);
 }
 
 // ---------------------------------------------------------------------------
@@ -434,13 +440,13 @@ __device__ __forceinline__ void split_finish(const BwdArgs &a, floatx16 (&dk)[D 
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         dk[d][i] = mul_then_add(dk[d][i], a.sm_scale, load_agent(other + (16 * d + i) * LANES));
-    store_row<E, D>(dk_row, dk, 1.0f, g);
+    store_row<E, D>(dk_row, dk, 1.0f, g, a.cols);
 #pragma unroll
     for (int d = 0; d < D / 32; ++d)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         dv[d][i] = mul_then_add(dv[d][i], 1.0f, load_agent(other + (HALF + 16 * d + i) * LANES));
-    store_row<E, D>(dv_row, dv, 1.0f, g);
+    store_row<E, D>(dv_row, dv, 1.0f, g, a.cols);
   }
 }
 
@@ -621,13 +627,13 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   if constexpr (T::KV_LDS) {
     // the workgroup's BK keys into LDS (zeros past Sk)
     DmaStager<D, KVSW, BK, T::NW> stk, stv;
-    stk.init(w, lane, a.k.ss);
-    stv.init(w, lane, a.v.ss);
-    stk.load(s_k, a.k.head(b, hk), a.k.ss, k0, Sk, w);
-    stv.load(s_v, a.v.head(b, hk), a.v.ss, k0, Sk, w);
+    stk.init(w, lane, a.k.ss, a.cols);
+    stv.init(w, lane, a.v.ss, a.cols);
+    stk.load(s_k, a.k.head(b, hk), a.k.ss, k0, Sk, w, a.cols);
+    stv.load(s_v, a.v.head(b, hk), a.v.ss, k0, Sk, w, a.cols);
   } else {
-    load_row_frags<E, D>(kf, a.k.head(b, hk), a.k.ss, key, Sk, g);
-    load_row_frags<E, D>(vf, a.v.head(b, hk), a.v.ss, key, Sk, g);
+    load_row_frags<E, D>(kf, a.k.head(b, hk), a.k.ss, key, Sk, g, a.cols);
+    load_row_frags<E, D>(vf, a.v.head(b, hk), a.v.ss, key, Sk, g, a.cols);
   }
   // B operands of S and dP: K^T / V^T fragments K[key][16cc + 8g .. +7]
   // (registers, or LDS rows 32kg + l32 read like the query tiles' A rows)
@@ -671,8 +677,8 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   // s_dl = -delta.  Seeding the S and dP MFMAs with them yields
   // ck * s - LSE' and dP - delta with no per-score VALU work.
   DmaStager<D, QSW, BQ, T::NW> stq, stg;
-  stq.init(w, lane, a.q.ss);
-  stg.init(w, lane, a.dout.ss);
+  stq.init(w, lane, a.q.ss, a.cols);
+  stg.init(w, lane, a.dout.ss, a.cols);
   const float lse_mul = a.lse_mul;
   float lse_r = 0.0f, dl_r = 0.0f;   // raw LSE / delta of row m0 + tid
   // Q and dO go straight to LDS stage `st`; LSE / delta through VGPRs.
@@ -697,8 +703,8 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
   RowCursor cq, cg;
   kfloat *rm_h;
   auto aim = [&](int h, int m0) {
-    cq.init(a.q.head(b, h), a.q.ss, m0, Sq, D, BQ);
-    cg.init(a.dout.head(b, h), a.dout.ss, m0, Sq, D, BQ);
+    cq.init(a.q.head(b, h), a.q.ss, m0, Sq, mem_cols<D>(a.cols), BQ);
+    cg.init(a.dout.head(b, h), a.dout.ss, m0, Sq, mem_cols<D>(a.cols), BQ);
     rm_h = (kfloat *)(a.rmax + ((int64_t)b * a.H + h) * ng * 2);
   };
   aim(cur_h, cur_m0);
@@ -1135,8 +1141,10 @@ __device__ __forceinline__ void dkdv_block(const BwdArgs &a, const int bid, f16 
       store_row_f32<D>(p + (int64_t)BHk * Sk * D, dv, 1.0f, g);
       return;
     }
-    store_row<E, D>(a.dk + b * a.dk_sb + hk * a.dk_sh + (int64_t)key * a.dk_ss, dk, dk_mul, g);
-    store_row<E, D>(a.dv + b * a.dv_sb + hk * a.dv_sh + (int64_t)key * a.dv_ss, dv, 1.0f, g);
+    store_row<E, D>(a.dk + b * a.dk_sb + hk * a.dk_sh + (int64_t)key * a.dk_ss, dk, dk_mul, g,
+                    a.cols);
+    store_row<E, D>(a.dv + b * a.dv_sb + hk * a.dv_sh + (int64_t)key * a.dv_ss, dv, 1.0f, g,
+                    a.cols);
   }
 }
 
@@ -1151,6 +1159,7 @@ __global__ __launch_bounds__(256) void fa_bwd_seg_sum_kernel(BwdArgs a) {
   if (i >= rows * (D / 4)) return;
   const int64_t row = i / (D / 4);
   const int c = 4 * (int)(i % (D / 4));
+  if (past_cols<D>(c, a.cols)) return;
   const float *p = a.seg_part + (int64_t)blockIdx.y * rows * D + row * D + c;
   floatx4 acc = *(const floatx4 *)p;
 #pragma unroll 4
@@ -1251,8 +1260,8 @@ __device__ __forceinline__ void dq_block(const BwdArgs &a, const int bid, f16 *s
   const f16 *vb = a.v.head(b, hk);
 
   vec8<E> qf[D / 16], gf[D / 16];
-  load_row_frags<E, D>(qf, a.q.head(b, h), a.q.ss, qrow, Sq, g);
-  load_row_frags<E, D>(gf, a.dout.head(b, h), a.dout.ss, qrow, Sq, g);
+  load_row_frags<E, D>(qf, a.q.head(b, h), a.q.ss, qrow, Sq, g, a.cols);
+  load_row_frags<E, D>(gf, a.dout.head(b, h), a.dout.ss, qrow, Sq, g, a.cols);
 
   int kv_end = Sk;
   if (CAUSAL) kv_end = min(Sk, q0 + BM + off);
@@ -1266,17 +1275,17 @@ __device__ __forceinline__ void dq_block(const BwdArgs &a, const int bid, f16 *s
 
   // K and V tiles go straight to LDS (fa_common.hpp DmaStager).
   DmaStager<D, SW_AT, BN, NW> stk, stv;
-  stk.init(w, lane, a.k.ss);
-  stv.init(w, lane, a.v.ss);
+  stk.init(w, lane, a.k.ss, a.cols);
+  stv.init(w, lane, a.v.ss, a.cols);
   auto load_tile = [&](int n0, auto stc) {
-    stk.load(k_st(stc), kb, a.k.ss, n0, Sk, w);
-    stv.load(v_st(stc), vb, a.v.ss, n0, Sk, w);
+    stk.load(k_st(stc), kb, a.k.ss, n0, Sk, w, a.cols);
+    stv.load(v_st(stc), vb, a.v.ss, n0, Sk, w, a.cols);
   };
   // the loop loads tile t + 1 during tile t: cursors from tile t_lo + 1,
   // advanced by a tile per load
   RowCursor ck, cv;
-  ck.init(kb, a.k.ss, (t_lo + 1) * BN, Sk, D, BN);
-  cv.init(vb, a.v.ss, (t_lo + 1) * BN, Sk, D, BN);
+  ck.init(kb, a.k.ss, (t_lo + 1) * BN, Sk, mem_cols<D>(a.cols), BN);
+  cv.init(vb, a.v.ss, (t_lo + 1) * BN, Sk, mem_cols<D>(a.cols), BN);
   auto load_next = [&](auto stc) {
     stk.load(k_st(stc), ck.rsrc(), w);
     stv.load(v_st(stc), cv.rsrc(), w);
@@ -1304,7 +1313,7 @@ __device__ __forceinline__ void dq_block(const BwdArgs &a, const int bid, f16 *s
     // delta = rowsum(O * dO) from the lane's half row and its lane ^ 32
     // partner's (the pre-pass, folded in); the dK/dV kernel reads it later
     vec8<E> of[D / 16];
-    load_row_frags<E, D>(of, a.o.head(b, h), a.o.ss, qrow, Sq, g);
+    load_row_frags<E, D>(of, a.o.head(b, h), a.o.ss, qrow, Sq, g, a.cols);
     float acc = 0.0f;
 #pragma unroll
     for (int c = 0; c < D / 16; ++c)
@@ -1476,7 +1485,8 @@ __device__ __forceinline__ void dq_block(const BwdArgs &a, const int bid, f16 *s
     return;
   }
   if (qrow < Sq)
-    store_row<E, D>(a.dq + b * a.dq_sb + h * a.dq_sh + (int64_t)qrow * a.dq_ss, dq, dq_mul, g);
+    store_row<E, D>(a.dq + b * a.dq_sb + h * a.dq_sh + (int64_t)qrow * a.dq_ss, dq, dq_mul, g,
+                    a.cols);
 }
 
 template <typename E, int D, bool CAUSAL, int SPLIT, bool PRE = false, int NW = 4>

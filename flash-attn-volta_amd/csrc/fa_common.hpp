@@ -196,6 +196,7 @@ struct RowCursor {
   int left;           // rows S - r
   int rows_step;      // rows per step
 
+  // (D: the columns of a row in memory)
   __device__ __forceinline__ void init(const f16 *head, int64_t ss, int r, int S, int D,
                                        int rows) {
     base = reinterpret_cast<const char *>(head + (int64_t)r * ss);
@@ -339,6 +340,21 @@ __host__ __device__ __forceinline__ constexpr int lds_row(int r) {
   return SW == SW_PD ? r * D + 8 * ((r * D) >> 9) : r * D;
 }
 
+// Rows of 16 columns run in the D = 32 kernels (`cols` = 16 in their
+// arguments): the tile loads, fragments and stores leave out columns 16-31,
+// which are zeros on the chip and absent in memory.  Copying such tensors
+// to 32 columns and back instead took 240 us a step at (4,256,4,16), whose
+// kernels take 20.  past_cols: true for columns that are not there; mem_cols:
+// the columns that are (a constant but for D = 32).
+template <int D>
+__device__ __forceinline__ constexpr bool past_cols(int col, int cols) {
+  return D == 32 && col >= cols;
+}
+template <int D>
+__device__ __forceinline__ constexpr int mem_cols(int cols) {
+  return D == 32 ? cols : D;
+}
+
 typedef __attribute__((address_space(3))) void lds_void;
 
 // One buffer_load_dwordx4 ... lds: lane i's 16 bytes at byte offset `voff`
@@ -358,17 +374,20 @@ struct DmaStager {
   static_assert(PER_WAVE >= 1, "tile smaller than one DMA instruction per wave");
   int off[PER_WAVE];   // global byte offset of this lane's chunk, relative to row r0
 
-  __device__ __forceinline__ void init(int w, int lane, int64_t ss) {
+  __device__ __forceinline__ void init(int w, int lane, int64_t ss, int cols = D) {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       const int byte = (w * PER_WAVE + j) * 1024 + 16 * lane;
       const int p = byte / (2 * D), pc = (byte % (2 * D)) / 16;
       off[j] = kperm_row(p) * (int)ss * 2 + 16 * (pc ^ swz<D, SW>(p));
+      // absent columns: past any extent of such a tensor (under 2^31 bytes a
+      // head, checked by the host), so they load zeros
+      if (past_cols<D>(8 * (pc ^ swz<D, SW>(p)), cols)) off[j] = INT32_MIN;
     }
   }
   __device__ __forceinline__ void load(f16 *slot, const f16 *head, int64_t ss, int r0, int S,
-                                       int w) const {
-    load(slot, rows_rsrc(head, ss, r0, S, D), w);
+                                       int w, int cols = D) const {
+    load(slot, rows_rsrc(head, ss, r0, S, mem_cols<D>(cols)), w);
   }
   __device__ __forceinline__ void load(f16 *slot, __amdgpu_buffer_rsrc_t rs, int w) const {
     // one KiB per instruction, plus SW_PD's 16 bytes after each

@@ -57,6 +57,7 @@ struct FwdArgs {
   int n_qtiles;
   float c;             // |sm_scale| * log2(e), clamped away from 0
   int neg;             // 1 when sm_scale < 0: Q is negated on load
+  int cols;            // columns of a row in memory: D, or 16 with D = 32 (past_cols)
   int zigzag;          // causal tile order: 1 zigzag heavy / light, 0 heaviest first
   // split-KV mode only (fa_fwd_kernel<..., SPLITKV = true>):
   int kv_split;        // keys per split, a multiple of the 64-key tile
@@ -267,16 +268,16 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
   // in kperm row order, chunks swizzled; rows past Sk read as zeros.
   DmaStager<D, SW_A, BN, NW> stk;   // K: read only as A operands
   DmaStager<D, SW_T, BN, NW> stv;   // V: read only transposed
-  stk.init(w, lane, a.k.ss);
-  stv.init(w, lane, a.v.ss);
-  auto load_k = [&](int n0, auto sc) { stk.load(k_sl(sc), kb, a.k.ss, n0, Sk, w); };
+  stk.init(w, lane, a.k.ss, a.cols);
+  stv.init(w, lane, a.v.ss, a.cols);
+  auto load_k = [&](int n0, auto sc) { stk.load(k_sl(sc), kb, a.k.ss, n0, Sk, w, a.cols); };
   // Iteration t loads K(t + 2) and V(t) (the prologue K(0), K(1) and, at
   // D = 128, V(0)):
   // cursors at those rows, each advanced by a tile per load (no per-tile
   // 64-bit multiplies).
   RowCursor ck, cv;
-  ck.init(kb, a.k.ss, 2 * BN, Sk, D, BN);
-  cv.init(vb, a.v.ss, 0, Sk, D, BN);
+  ck.init(kb, a.k.ss, 2 * BN, Sk, mem_cols<D>(a.cols), BN);
+  cv.init(vb, a.v.ss, 0, Sk, mem_cols<D>(a.cols), BN);
   auto load_k_next = [&](auto sc) {
     stk.load(k_sl(sc), ck.rsrc(), w);
     ck.advance();
@@ -395,7 +396,8 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
     const f16 *qp = (SPLITKV ? a.q.head(b, hk * grp + qr % grp) + (int64_t)(qr / grp) * a.q.ss
                              : a.q.head(b, h) + (int64_t)qr * a.q.ss) + 8 * g;
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c) qf[c] = ld8<E>(qp + 16 * c);
+    for (int c = 0; c < D / 16; ++c)
+      qf[c] = past_cols<D>(16 * c, a.cols) ? vec8<E>{} : ld8<E>(qp + 16 * c);
     if (pre) {
 #pragma unroll
       for (int c = 0; c < D / 16; ++c)
@@ -812,6 +814,7 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         vec4<E> v4;
+        if (past_cols<D>(c_row(4 * r, g), a.cols)) continue;
 #pragma unroll
         for (int j = 0; j < 4; ++j) v4[j] = (E)(oacc[d][4 * r + j] * inv);
         *(vec4<E> *)(orow + 32 * d + c_row(4 * r, g)) = v4;
@@ -842,6 +845,7 @@ struct CombineArgs {
   float *lse;                       // (B, H, Sq) or nullptr
   int B, Sq, H, n_splits;
   int zgroups;                      // power of two, at most 256 / (D / 8)
+  int cols;                         // columns of an O row in memory (FwdArgs)
   // pair mode: the forward's tile rows (0: split-KV layout), query tiles
   // per (b, h), key tile and causal offset
   int pair_bm, nb, bn, Sk, off;
@@ -932,7 +936,8 @@ __global__ __launch_bounds__(256) void fa_fwd_combine_kernel(CombineArgs a) {
   vec8<E> out;
 #pragma unroll
   for (int i = 0; i < 8; ++i) out[i] = (E)(o8[i] * inv);
-  *(vec8<E> *)(a.o + b * a.o_sb + s * a.o_ss + hh * a.o_sh + 8 * j) = out;
+  if (!past_cols<D>(8 * j, a.cols))
+    *(vec8<E> *)(a.o + b * a.o_sb + s * a.o_ss + hh * a.o_sh + 8 * j) = out;
   if (a.lse != nullptr && j == 0)
     a.lse[bh * a.Sq + s] = tot > 0.0f ? (mt + fast_log2(tot)) * kLn2 : kPosInf;
 }

@@ -124,7 +124,8 @@ struct FlashAttnFn : public torch::autograd::Function<FlashAttnFn> {
                         int64_t handle, bool split) {
     const Plan &p = *reinterpret_cast<const Plan *>(handle);
     const c10::DeviceGuard guard(q.device());
-    Tensor out = at::empty({p.B, p.Sq, p.H, p.D}, q.options());
+    // (head_dim 16 runs as half of p.D = 32)
+    Tensor out = at::empty({p.B, p.Sq, p.H, q.size(3)}, q.options());
     Tensor lse = at::empty({p.B, p.H, p.Sq}, q.options().dtype(at::kFloat));
     void *stream = stream_of(q);
     if (p.fwd_ws) {
@@ -165,10 +166,10 @@ struct FlashAttnFn : public torch::autograd::Function<FlashAttnFn> {
       dout = dout.clone(at::MemoryFormat::Contiguous);
       std::copy(p.o_st, p.o_st + 4, do_st);
     }
-    Tensor dq = at::empty({p.B, p.Sq, p.H, p.D}, q.options());
+    Tensor dq = at::empty({p.B, p.Sq, p.H, q.size(3)}, q.options());
     // separate allocations, as the Python path's
-    Tensor dk = at::empty({p.B, p.Sk, p.Hk, p.D}, q.options());
-    Tensor dv = at::empty({p.B, p.Sk, p.Hk, p.D}, q.options());
+    Tensor dk = at::empty({p.B, p.Sk, p.Hk, q.size(3)}, q.options());
+    Tensor dv = at::empty({p.B, p.Sk, p.Hk, q.size(3)}, q.options());
     const size_t nb = split ? p.ws_split : p.ws_plain;
     Tensor ws = at::empty({(int64_t)nb}, q.options().dtype(at::kByte));
     void *stream = stream_of(q);

@@ -37,6 +37,7 @@ NOALLOC_SCRATCH_BYTES = 64 << 20
 # element types (enum fa_dtype)
 FA_DTYPE_F16 = 0
 FA_DTYPE_BF16 = 1
+FA_HALF_COLS = 0x100
 
 # Every symbol include/fa_mi355x.h declares.
 EXPORTED_SYMBOLS = (

@@ -6,7 +6,7 @@ value.  One ``fa_bwd`` call (include/fa_mi355x.h) runs two gfx950 kernels
 on the current stream: the dQ kernel, which also computes
 delta = rowsum(dO * O) (the reference's separate pre-pass) into the
 caller-owned workspace, then the dK/dV kernel, which reads it.  No permute
-copies; D = 16 is zero-padded to 32 like the forward.
+copies; D = 16 runs on its 16 columns like the forward.
 """
 from __future__ import annotations
 
@@ -19,7 +19,8 @@ from . import _capi, _runtime
 from ._runtime import VP
 from .forward import (_DTYPES, _GENERIC, _MAX_PLANS, NATIVE_HEAD_DIMS, SUPPORTED_HEAD_DIMS,
                       _check_gqa, _contiguous_strides, _kernel_ready, _layout_ready, _on_device,
-                      _pad_d, _require, _stream_ptr, _strides_c, kernel_strides)
+                      _pad_d, _require, _stream_ptr, _strides_c, kernel_dims, kernel_strides,
+                      planned_dim)
 
 
 def flash_attn_backward(
@@ -92,7 +93,7 @@ def backward_planned(do, q, k, v, o, lse, causal, sm_scale, gqa):
         (_validate_bwd_gqa if gqa else _validate_bwd)(do, q, k, v, o, lse)
         plan = _GENERIC
         B, N, H, D = q.shape
-        if (D in NATIVE_HEAD_DIMS and q.numel() and k.numel() and lse.is_contiguous()
+        if (planned_dim(do, q, k, v, o) and q.numel() and k.numel() and lse.is_contiguous()
                 and all(_layout_ready(t) for t in (do, q, k, v, o))):
             plan = _BwdPlan(B, N, k.shape[1], H, k.shape[2], D,
                             [kernel_strides(t) for t in (do, q, k, v, o)], q.stride(), k.stride(),
@@ -124,7 +125,10 @@ class _BwdPlan:
     def __init__(self, B, Sq, Sk, H, Hk, D, in_strides, q_stride, k_stride, dtype, device,
                  causal, sm_scale, gqa):
         lib = _capi.load()
-        self.q_shape, self.k_shape = (B, Sq, H, D), (B, Sk, Hk, D)
+        cols = D
+        D, code = kernel_dims(D, dtype)
+        gqa = gqa or D != cols      # the entry point that takes any dtype code
+        self.q_shape, self.k_shape = (B, Sq, H, cols), (B, Sk, Hk, cols)
         q_st, k_st = _contiguous_strides(self.q_shape), _contiguous_strides(self.k_shape)
         self.q_like, self.k_like = tuple(q_stride) == q_st, tuple(k_stride) == k_st
         self.dtype, self.device, self.idx = dtype, device, device.index
@@ -139,7 +143,7 @@ class _BwdPlan:
         if gqa:
             self.name = "fa_bwd_gqa"
             self.rest = _runtime.convert(self.name, 11, (B, Sq, Sk, H, Hk, D, *st, float(sm_scale),
-                                                         c, _DTYPES[dtype]))
+                                                         c, code))
         else:
             self.name = "fa_bwd"
             self.rest = _runtime.convert(self.name, 11, (B, Sq, H, D, *st, float(sm_scale), c))

@@ -7,8 +7,10 @@ arity, layouts and the +inf LSE rule for rows that see no key
 kernel behind ``fa_fwd`` (include/fa_mi355x.h); the (B, S, H, D) strides go
 straight to the kernel, so there are no permute copies, and D = 32 / 64 / 128
 run natively with no padding.  D = 16, which the reference also accepts
-(triton_fa.py:317), is zero-padded to 32 here (an on-device copy; the padded
-columns contribute exactly zero to every dot product).
+(triton_fa.py:317), runs in the D = 32 kernels on its 16 columns
+(FA_HALF_COLS); only layouts they cannot read are zero-padded to 32 (an
+on-device copy; the padded columns contribute exactly zero to every dot
+product).
 """
 from __future__ import annotations
 
@@ -56,6 +58,22 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     if t.data_ptr() % 16 == 0 and (t.is_contiguous() or _layout_ready(t)):
         return t            # contiguous: D is a multiple of 8, so every stride is too
     return t.clone(memory_format=torch.contiguous_format)
+
+
+def kernel_dims(D: int, dtype):
+    """(D, dtype code) with which the C ABI takes head_dim D: 16 columns run
+    as half of D = 32."""
+    if D == 16:
+        return 32, _DTYPES[dtype] | _capi.FA_HALF_COLS
+    return D, _DTYPES[dtype]
+
+
+def planned_dim(*tensors) -> bool:
+    """The kernels take these (B, S, heads, D) tensors' head_dim without
+    padding: a native one, or 16 with heads of under 2^31 bytes."""
+    D = tensors[0].size(3)
+    return D in NATIVE_HEAD_DIMS or (D == 16 and all(
+        (t.size(1) - 1) * t.stride(1) * 2 + 64 < 2 ** 31 for t in tensors))
 
 
 _STRIDES = {}
@@ -192,12 +210,12 @@ def forward_planned(q, k, v, causal, sm_scale, want_lse, gqa):
 
 class _FwdPlan:
     """Launch plan of one forward call signature whose tensors the kernels
-    read in place (native head_dim, ready layouts, nothing empty): the C
+    read in place (head_dim, ready layouts, nothing empty): the C
     entry point and its size / stride / scale / flag arguments, converted
     once.  A call allocates out (and LSE) and passes the data pointers and
     the current stream; the general path (_forward) gives the same
     results."""
-    __slots__ = ("fn", "name", "args", "out_shape", "lse_shape", "dtype", "device", "idx",
+    __slots__ = ("fn", "name", "args", "out_shape", "lse_shape", "dtype", "code", "device", "idx",
                  "like", "ws_bytes", "causal", "sm_scale", "gqa", "sizes", "st", "q_stride",
                  "k_stride", "bwd", "cpp")
 
@@ -205,15 +223,16 @@ class _FwdPlan:
     def build(cls, q, k, v, causal, sm_scale, want_lse, gqa):
         B, Sq, H, D = q.shape
         Sk, Hk = k.shape[1], k.shape[2]
-        if (D not in NATIVE_HEAD_DIMS or q.numel() == 0 or Sk == 0
+        if (not planned_dim(q, k, v) or q.numel() == 0 or Sk == 0
                 or not (_layout_ready(q) and _layout_ready(k) and _layout_ready(v))):
             return None
         p = cls()
         p.causal = bool(causal)
-        p.sm_scale = float(1.0 / math.sqrt(D) if sm_scale is None else sm_scale)
-        p.gqa = gqa
-        p.dtype, p.device, p.idx = q.dtype, q.device, q.device.index
+        p.sm_scale = float(1.0 / math.sqrt(q.shape[3]) if sm_scale is None else sm_scale)
         p.out_shape = (B, Sq, H, D)
+        D, p.code = kernel_dims(D, q.dtype)
+        p.gqa = gqa = gqa or D != q.shape[3]     # the entry points that take any dtype code
+        p.dtype, p.device, p.idx = q.dtype, q.device, q.device.index
         p.lse_shape = (B, H, Sq) if want_lse else None
         o_st = _contiguous_strides(p.out_shape)
         p.like = q.stride() == o_st          # empty_like(q) is then contiguous
@@ -221,18 +240,17 @@ class _FwdPlan:
         p.sizes, p.st, p.q_stride, p.k_stride = (B, Sq, Sk, H, Hk, D), st, q.stride(), k.stride()
         p.bwd = None
         p.cpp = 0
-        dt = _DTYPES[q.dtype]
         # the schedule with a workspace (split-KV for decode shapes, the
         # balanced causal one for square one-round causal grids), if any
         p.ws_bytes = int(_capi.load().fa_fwd_workspace_bytes(B, Sq, Sk, H, Hk, D, int(p.causal)))
         if p.ws_bytes:
             p.name = "fa_fwd_ws"
             p.args = _runtime.convert(p.name, 6, (p.ws_bytes, B, Sq, Sk, H, Hk, D, *st,
-                                                  p.sm_scale, int(p.causal), dt))
+                                                  p.sm_scale, int(p.causal), p.code))
         elif gqa:
             p.name = "fa_fwd_gqa"
             p.args = _runtime.convert(p.name, 5, (B, Sq, Sk, H, Hk, D, *st, p.sm_scale,
-                                                  int(p.causal), dt))
+                                                  int(p.causal), p.code))
         else:
             p.name = "fa_fwd"
             p.args = _runtime.convert(p.name, 5, (B, Sq, H, D, *st, p.sm_scale, int(p.causal)))
@@ -263,7 +281,7 @@ class _FwdPlan:
         q, k, v are this plan's, out and dO contiguous."""
         from .backward import _BwdPlan
         q, k, v, o = self.st
-        self.bwd = _BwdPlan(*self.sizes, (o, q, k, v, o), self.q_stride, self.k_stride, self.dtype,
+        self.bwd = _BwdPlan(*self.sizes[:5], self.out_shape[3], (o, q, k, v, o), self.q_stride, self.k_stride, self.dtype,
                             self.device, self.causal, self.sm_scale, self.gqa)
         return self.bwd
 
@@ -273,9 +291,10 @@ class _FwdPlan:
         strides, contiguous dQ and dK strides, and the workspace sizes."""
         B, Sq, Sk, H, Hk, D = self.sizes
         lib = _capi.load()
-        dq_st = _strides_c((B, Sq, H, D), _contiguous_strides((B, Sq, H, D)))
-        dk_st = _strides_c((B, Sk, Hk, D), _contiguous_strides((B, Sk, Hk, D)))
-        ints = [B, Sq, Sk, H, Hk, D, int(self.gqa), int(self.causal), _DTYPES[self.dtype]]
+        k_shape = (B, Sk, Hk, self.out_shape[3])
+        dq_st = _strides_c(self.out_shape, _contiguous_strides(self.out_shape))
+        dk_st = _strides_c(k_shape, _contiguous_strides(k_shape))
+        ints = [B, Sq, Sk, H, Hk, D, int(self.gqa), int(self.causal), self.code]
         for arr in (*self.st, dq_st, dk_st):
             ints += list(arr)
         ints += [self.ws_bytes,

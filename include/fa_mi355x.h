@@ -72,6 +72,13 @@ enum fa_dtype {
   FA_DTYPE_BF16 = 1           /* bfloat16                                   */
 };
 
+/* Or-ed into the dtype of fa_fwd_gqa, fa_fwd_ws and fa_bwd_gqa with D = 32:
+ * every row holds 16 columns, and columns 16-31 are taken as zeros and not
+ * stored (head_dim 16 without copies; sm_scale is the caller's as always).
+ * A head's rows then span under 2^31 bytes, else FA_ERR_TOO_LARGE; with any
+ * other D, FA_ERR_HEAD_DIM.  The workspace sizes are those of D = 32. */
+#define FA_HALF_COLS 0x100
+
 /* Version of this ABI (FA_ABI_VERSION of the build). */
 int fa_abi_version(void);
 
