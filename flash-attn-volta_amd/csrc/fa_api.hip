@@ -628,12 +628,15 @@ SplitPlan splitkv_plan(const Shape &s) {
 //     packed, 5.3 TB/s, a large copy's rate; (64, 4, 4000, 32 / 8, 128)
 //     595 -> 179 us);
 //   * chunks: any short block of queries whose plain grid leaves CUs idle.
-//     The model below prices both: a CU runs one 64 x 64 tile step in `step`
-//     us whether one workgroup or two share it, a packed launch adds about
-//     8 us of start-up and merge and the partials' traffic.  Measured, bf16
-//     (1, Sq, 8448 keys, 32 / 8, 128): Sq = 256 90 -> 52 us, 128 92 -> 32,
-//     32 92 -> 19; from Sq = 512 on (one plain workgroup per CU) splitting
-//     gains nothing and the model keeps the plain grid.
+//     The model below prices both in us: a workgroup's 64 x 64 tile step
+//     takes `lone` alone on its CU and grows with the workgroups per CU
+//     from where they fill it; a workgroup's start-up; and for a split the
+//     merge launch and its partials' traffic.  Measured, bf16, plain ->
+//     chosen: (1, Sq, 8448 keys, 32 / 8, 128) Sq = 256 90 -> 52 us, 128 92 ->
+//     32, 32 92 -> 19, 400 of 9000 95 -> 75, 200 of 3000 36 -> 27, (2,64,2000)
+//     28 -> 20; (1,1000,9000,14/2,64) 67 -> 50; against it (1,600,3000,32/8,128)
+//     44 -> 56, (1,300,2000,28/4,128) 27.5 -> 28.5 and (1,200,1000,32/32,128)
+//     16.0 -> 18.6 in two ranges, which the model leaves plain.
 SplitPlan fwd_split_plan(const Shape &s, int causal) {
   const SplitPlan none{0, 0};
   const int64_t grp = s.H / s.Hk;
@@ -647,17 +650,18 @@ SplitPlan fwd_split_plan(const Shape &s, int causal) {
   // (a causal grid's plain sweeps must be near the full length: at least
   // half of the keys lie before the block)
   if (causal && (int64_t)s.Sk < 2 * (int64_t)s.Sq) return none;
-  const double step = s.D >= 128 ? 0.6 : 0.35;
+  const double lone = s.D >= 128 ? 0.65 : 0.47, fill = s.D >= 128 ? 0.9 : 0.75;
+  const double start = 6.0;
+  auto sweep_us = [&](int64_t wgs, int64_t tiles) {
+    const double w = fill * (double)wgs / (double)cus;
+    return lone * (w > 1.0 ? w : 1.0) * (double)tiles + start;
+  };
   const int64_t tiles = (s.Sk + 63) / 64, packed = packed_tiles(s);
-  const double t_plain = (double)((plain + cus - 1) / cus) * tiles * step;
-  double best = 0.85 * t_plain;
+  double best = 0.88 * sweep_us(plain, tiles);
   int64_t best_n = 0;
-  for (int64_t k = 1; k <= 8; ++k) {
-    const int64_t n = k * cus / packed < tiles / 4 ? k * cus / packed : tiles / 4;
-    if (n < 2) continue;
-    const int64_t t = (tiles + n - 1) / n;
+  for (int64_t n = 2; n <= 32 && 4 * n <= tiles; ++n) {
     const double rows = (double)s.B * s.H * s.Sq * n;
-    const double c = (double)((packed * n + cus - 1) / cus) * t * step + 8.0 +
+    const double c = sweep_us(packed * n, (tiles + n - 1) / n) + 2.0 + n +
                      rows * (s.D + 1) * 8.0 / 5.0e6;
     if (c < best) {
       best = c;
@@ -1199,6 +1203,11 @@ void bwd_plans(const Shape &s, int causal, DkdvSplit &plan, DqSplit &qplan) {
   plan = bwd_fused(s, causal, qplan) ? DkdvSplit{} : dkdv_split_plan(s, causal);
 }
 
+// one segment's fp32 dK and dV
+size_t segment_bytes(const Shape &s) {
+  return (size_t)2 * s.B * s.Hk * (size_t)s.Sk * s.D * sizeof(float);
+}
+
 // Sweep segments of the dK/dV blocks (fa::BwdArgs::seg_n), given the room
 // (fa_bwd_best_workspace_bytes).  A key block's sweep covers every query
 // head of its group, so few key/value heads leave few, long workgroups:
@@ -1207,11 +1216,13 @@ void bwd_plans(const Shape &s, int causal, DkdvSplit &plan, DqSplit &qplan) {
 // by the sum) and a workgroup's start-up, so as few as fill the GPU.
 // Measured, the backward (1 segment -> chosen), causal, D = 128:
 //   (1,4000,28/4) 762 -> 444 us (2; 4: 444, 8: 469), (1,3000,28/4) 563 -> 272
-//   (3), (1,2048,16/2) 428 -> 91 (8), (1,1024,32/8) 121 -> 62 (4),
-//   (1,512,32/8) 67 -> 40 (3), (1,3500,32/8) 411 -> 388 (2), (1,4096,32/8)
+//   (3), (1,2048,16/2) 428 -> 91 (8), (1,1024,32/8) 121 -> 62 (3), (1,700,64/8)
+//   162 -> 65 (4; 6: 72), (1,512,32/8) 67 -> 35 (4; 6: 40), (1,300,28/4) 72 -> 31
+//   (8), (1,128,28/4) 37 -> 24 (7), (1,3500,32/8) 411 -> 388 (2), (1,4096,32/8)
 //   (one full round, 256-tile sweeps) 510 -> 487 (2), but (1,4096,16/8) (one
 //   round, 128 tiles) +6 % and (2,3000,16/8) (1.5 rounds) +11 % with 2;
-// D = 64: (1,4096,14/2) 396 -> 134 (8), (1,2048,32/8) 131 -> 89 (4);
+// D = 64: (1,4096,14/2) 396 -> 134 (8), (1,3000,14/2) 300 -> 80 (8; 11: 89),
+//   (1,2048,32/8) 131 -> 84 (3), (1,700,14/2) 78 -> 24 (13);
 // equal heads: (1,2048,4/4) 65 -> 55, (2,1500,4/4) 54 -> 48 (2), but
 //   (1,2048,8/8) +6 %;
 // not causal: (1,2048,32/4,128) 467 -> 254 (4), (1,3000,32/8,128) 754 -> 529
@@ -1235,22 +1246,26 @@ int dkdv_segments(const Shape &s, int causal) {
     }
     return (int)best;
   }
+  if (blocks > slots) return 1;
   if (grp == 1) {
+    if (s.D != 128 || 8 * blocks > 3 * slots || sweep < 20) return 1;
     DkdvSplit plan;
     DqSplit qplan;
     bwd_plans(s, causal, plan, qplan);
-    return s.D == 128 && 8 * blocks <= 3 * slots && sweep >= 20 && qplan.split == 0 ? 2 : 1;
+    return qplan.split == 0 ? 2 : 1;
   }
-  if (blocks > slots) return 1;
   int64_t n = (slots + blocks - 1) / blocks;
   if (n < 2 && sweep >= 192) n = 2;
-  if (n > sweep / 10) n = sweep / 10;
+  // short sweeps: fewer than fill every slot, of at least 8 tiles -- or, while
+  // the partials stay under 10 MB, of at least 2
+  if (n > 3 && sweep < (s.D >= 128 ? 200 : 400)) n = (7 * slots + 10 * blocks - 1) / (10 * blocks);
+  if (n > sweep / 8) n = sweep / 8;
+  const int64_t full = (slots + blocks - 1) / blocks;
+  int64_t cheap = (int64_t)10000000 / (int64_t)segment_bytes(s);
+  cheap = cheap < sweep / 2 ? cheap : sweep / 2;
+  cheap = cheap < full ? cheap : full;
+  if (n < cheap) n = cheap;
   return n < 2 ? 1 : (n > 16 ? 16 : (int)n);
-}
-
-// one segment's fp32 dK and dV
-size_t segment_bytes(const Shape &s) {
-  return (size_t)2 * s.B * s.Hk * (size_t)s.Sk * s.D * sizeof(float);
 }
 
 // two segments x BM rows x D fp32 per split query block
