@@ -1544,6 +1544,7 @@ Shape square(int B, int S, int H, int D) { return Shape{B, S, S, H, H, D, FA_DTY
 
 struct RopeShape {
   int B, S, H, Hk, D, dtype;
+  int dw_16;   // FA_DW_16: the norm weights' gradients in the element type
 };
 
 int check_rope_shape(const RopeShape &s) {
@@ -1609,14 +1610,21 @@ int launch_rope_fwd(const fa::RopeArgs &a, int64_t blocks, hipStream_t st) {
 }
 
 template <typename E, int D>
-int launch_rope_bwd(const fa::RopeArgs &a, int64_t blocks, float *dwq, float *dwk,
+int launch_rope_bwd(const fa::RopeArgs &a, int64_t blocks, void *dwq, void *dwk, bool dw_16,
                     hipStream_t st) {
   hipLaunchKernelGGL((fa::fa_rope_bwd_kernel<E, D>), dim3((unsigned)blocks, 2), dim3(fa::kRopeThreads),
                      0, st, a);
   int rc = launch_status();
   if (rc || (a.side[0].w == nullptr && a.side[1].w == nullptr)) return rc;
-  hipLaunchKernelGGL(fa::fa_rope_dw_reduce_kernel<D>, dim3(D / 16, 2), dim3(fa::kRopeReduceThreads), 0, st,
-                     a.side[0].partial, a.side[1].partial, dwq, dwk, (int)blocks);
+  const dim3 grid(D / 16, 2), threads(fa::kRopeReduceThreads);
+  if (dw_16)
+    hipLaunchKernelGGL((fa::fa_rope_dw_reduce_kernel<E, D>), grid, threads, 0, st,
+                       a.side[0].partial, a.side[1].partial, static_cast<E *>(dwq),
+                       static_cast<E *>(dwk), (int)blocks);
+  else
+    hipLaunchKernelGGL((fa::fa_rope_dw_reduce_kernel<float, D>), grid, threads, 0, st,
+                       a.side[0].partial, a.side[1].partial, static_cast<float *>(dwq),
+                       static_cast<float *>(dwk), (int)blocks);
   return launch_status();
 }
 
@@ -1682,7 +1690,7 @@ int run_rope_fwd(const void *q, const void *k, void *q_out, void *k_out, const v
 
 int run_rope_bwd(const void *dq_out, const void *dk_out, const void *q, const void *k,
                  const void *cos, const void *sin, const void *wq, const void *wk, float eps,
-                 void *dq, void *dk, float *dwq, float *dwk, void *workspace,
+                 void *dq, void *dk, void *dwq, void *dwk, void *workspace,
                  size_t workspace_bytes, const RopeShape &s, const int64_t *dqo_st,
                  const int64_t *dko_st, const int64_t *q_st, const int64_t *k_st,
                  const int64_t *dq_st, const int64_t *dk_st, const int64_t *cs_st, void *stream) {
@@ -1742,7 +1750,7 @@ int run_rope_bwd(const void *dq_out, const void *dk_out, const void *q, const vo
   a.eps = eps;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t blocks = rope_blocks(s, norm);
-  FA_ROPE_DISPATCH(launch_rope_bwd, s, a, blocks, dwq, dwk, st);
+  FA_ROPE_DISPATCH(launch_rope_bwd, s, a, blocks, dwq, dwk, s.dw_16 != 0, st);
 }
 
 }  // namespace
@@ -2037,7 +2045,8 @@ int fa_rope_qk_bwd(const void *dq_out, const void *dk_out, const void *q, const 
                    const int64_t cs_strides[2], int dtype, void *stream) {
   return run_rope_bwd(dq_out, dk_out, q, k, cos, sin, q_norm_weight, k_norm_weight, eps, dq, dk,
                       dq_norm_weight, dk_norm_weight, workspace, workspace_bytes,
-                      RopeShape{B, S, H, Hk, D, dtype}, dq_out_strides, dk_out_strides, q_strides,
+                      RopeShape{B, S, H, Hk, D, dtype & ~FA_DW_16, (dtype & FA_DW_16) != 0},
+                      dq_out_strides, dk_out_strides, q_strides,
                       k_strides, dq_strides, dk_strides, cs_strides, stream);
 }
 

@@ -306,18 +306,20 @@ __global__ __launch_bounds__(kRopeThreads) void fa_rope_bwd_kernel(RopeArgs a) {
     rope_bwd_side<E, D, false>(a, t);
 }
 
-// dw[side][d] = sum over nblk partials, in a fixed order.  Grid (D / 16, 2),
+// dw[side][d] = sum over nblk partials, in a fixed order, as OUT (fp32, or the
+// element type: a caller's cast of each would be a launch of its own, 2 of 5
+// in a normed step).  Grid (D / 16, 2),
 // 1024 threads: 16 columns x 64 interleaved partial subsets per workgroup,
 // the subsets' loads unrolled so that many are in flight, then a tree over
 // the 64 subsets in LDS.
 constexpr int kRopeReduceThreads = 1024;
 
-template <int D>
+template <typename OUT, int D>
 __global__ __launch_bounds__(kRopeReduceThreads) void fa_rope_dw_reduce_kernel(
-    const float *partial_q, const float *partial_k, float *dw_q, float *dw_k, int nblk) {
+    const float *partial_q, const float *partial_k, OUT *dw_q, OUT *dw_k, int nblk) {
   constexpr int SEGS = kRopeReduceThreads / 16;
   const float *part = blockIdx.y == 0 ? partial_q : partial_k;
-  float *dw = blockIdx.y == 0 ? dw_q : dw_k;
+  OUT *dw = blockIdx.y == 0 ? dw_q : dw_k;
   if (part == nullptr) return;
   __shared__ float s_acc[SEGS][17];
   const int c = threadIdx.x % 16, seg = threadIdx.x / 16;
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(kRopeReduceThreads) void fa_rope_dw_reduce_kernel(
     if (seg < w) s_acc[seg][c] += s_acc[seg + w][c];
     __syncthreads();
   }
-  if (seg == 0) dw[col] = s_acc[0][c];
+  if (seg == 0) dw[col] = (OUT)s_acc[0][c];
 }
 
 }  // namespace fa

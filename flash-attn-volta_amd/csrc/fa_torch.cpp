@@ -264,7 +264,7 @@ struct RopeFn : public torch::autograd::Function<RopeFn> {
       kernel_strides(x[i], x_st[i]);
       d[i] = at::empty(g[i].sizes(), opt);
       kernel_strides(d[i], d_st[i]);
-      if (s[4 + i].defined()) dw[i] = at::empty({g[i].size(3)}, opt.dtype(at::kFloat));
+      if (s[4 + i].defined()) dw[i] = at::empty({g[i].size(3)}, opt);   // the weight's dtype
     }
     table_strides(cos, cs);
     const int B = (int)g[0].size(0), S = (int)g[0].size(1), H = (int)g[0].size(2),
@@ -275,13 +275,12 @@ struct RopeFn : public torch::autograd::Function<RopeFn> {
     auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
     check(fa_rope_qk_bwd(g[0].data_ptr(), g[1].data_ptr(), x[0].data_ptr(), x[1].data_ptr(),
                          cos.data_ptr(), sin.data_ptr(), ptr(wq), ptr(wk), (float)eps,
-                         d[0].data_ptr(), d[1].data_ptr(), static_cast<float *>(ptr(dw[0])),
+                         d[0].data_ptr(), d[1].data_ptr(), static_cast<float *>(ptr(dw[0])),   // FA_DW_16
                          static_cast<float *>(ptr(dw[1])), ptr(ws),
                          ws.defined() ? (size_t)ws.numel() : 0, B, S, H, Hk, D, g_st[0], g_st[1],
-                         x_st[0], x_st[1], d_st[0], d_st[1], cs, dtype_of(cos), stream_of(cos)),
+                         x_st[0], x_st[1], d_st[0], d_st[1], cs, dtype_of(cos) | FA_DW_16,
+                         stream_of(cos)),
           "fa_rope_qk_bwd");
-    for (int i = 0; i < 2; ++i)
-      if (dw[i].defined()) dw[i] = dw[i].to(s[4 + i].scalar_type());
     return {d[0], d[1], Tensor(), Tensor(), dw[0], dw[1], Tensor()};
   }
 };

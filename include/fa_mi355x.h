@@ -425,6 +425,8 @@ int fa_rope_qk_fwd(const void *q, const void *k, void *q_out, void *k_out,
                    const int64_t q_out_strides[4], const int64_t k_out_strides[4],
                    const int64_t cs_strides[2], int dtype, void *stream);
 
+#define FA_DW_16 0x200
+
 /* Bytes of workspace fa_rope_qk_bwd needs when a norm weight is given (0 for
  * an invalid shape).  Depends only on the sizes. */
 size_t fa_rope_qk_workspace_bytes(int B, int S, int H, int Hk, int D);
@@ -432,7 +434,9 @@ size_t fa_rope_qk_workspace_bytes(int B, int S, int H, int Hk, int D);
 /*
  * Backward of fa_rope_qk_fwd: from the gradients of q_out / k_out, the
  * gradients of q / k, and for a normed side the gradient of its weight,
- * (D) fp32, reduced in a fixed order (reproducible).  q / k (the forward's
+ * (D) fp32, reduced in a fixed order (reproducible); with FA_DW_16 or-ed into
+ * dtype the fp32 sum is stored in the element type (dq_norm_weight /
+ * dk_norm_weight then point to 16-bit values).  q / k (the forward's
  * inputs), dq_norm_weight / dk_norm_weight and the workspace are read only
  * for a side with a norm weight and may be NULL otherwise.
  */
