@@ -265,6 +265,47 @@ bool dkdv_split2(int D, bool causal, int Sk, int64_t heads) {
   return D == 128 ? 2 * n <= cus : n < 2 * cus;
 }
 
+// The fused backward launch (fa::fa_bwd_fused_kernel) of a non-causal
+// problem: whether fa_bwd takes it in place of the dQ kernel (delta folded
+// in) then the dK/dV kernel, and its layouts.  Each of those two kernels ends
+// on a partly idle round and waits for the other; fused, the dQ blocks fill
+// the dK/dV blocks' tail, for one pre-pass over O and dO more.  `seg` is the
+// dK/dV blocks' sweep segments.  Measured, the backward, us, two kernels ->
+// fused:
+//   D = 64: on but for long key grids of one- or two-tile sweeps ((32, 100 x
+//     1500, 8) 93 / 97): (2,1000,25) 85 -> 65, (4,1500,12) 128 -> 109, (8,577,16)
+//     66 -> 59, (1,3000,6) 88 -> 70, (1,4096,26) 451 -> 388, (1,4096,16) 242 ->
+//     236, (16,197,12) 28.6 -> 23.1, (1,700,12) 27 -> 19; (32,197,12) 39.4 -> 40.7,
+//     (16,700,16) 151 -> 152.  Query-split dK/dV blocks under 1.2 workgroups per
+//     CU ((4,1000,8) 43 / 41, (16,197,12) 23 / 27), key-split dQ blocks under
+//     0.75 on sweeps of 8 tiles or more ((1,4096,4) 105 / 86, (4,512,12) 25 / 23,
+//     (4,1000,8) 41 / 45), both for single 64-row blocks.
+//   D = 32 (the same lines): (2,1000,25) 57 -> 42, (1,4096,16) 163 -> 145.
+//   D = 128, one eight-wave workgroup per CU: where every block has a CU of
+//     its own at once ((1,700,12) 42 -> 33, (1,2048,4) 77 -> 58, (1,1500,8) 73 ->
+//     54, (2,1000,10) 69 -> 53), or the dK/dV grid's last round is mostly empty
+//     and the sweeps are of 5 to 48 tiles ((4,1500,6) 166 -> 121, (1,3000,12)
+//     283 -> 239, (2,3000,12) 486 -> 421, (8,300,12) 57 -> 48); against it
+//     (1,4096,20) 668 / 687, (1,6000,12) 924 / 945, (16,512,12) 147 / 158,
+//     (20,197,12) 62 / 64, and in segments (1,3000,4) 105 / 118, (1,3000,32/8)
+//     537 / 554.
+struct NcFused {
+  bool on, kv2, q2;   // kv2, q2: the two-halves layouts of dK/dV and dQ
+};
+
+NcFused nc_fused(int B, int Sq, int Sk, int H, int Hk, int D, int seg) {
+  const int64_t cus = device_cus();
+  const int64_t nq = grid128(Sq, (int64_t)B * H), nkv = grid128(Sk, (int64_t)B * Hk * seg);
+  if (D <= 64)
+    return NcFused{!(Sq <= 128 && nkv >= 4 * cus), Sk <= 64 || (seg == 1 && 5 * nkv < 6 * cus),
+                   Sq <= 64 || (4 * nq <= 3 * cus && Sk >= 512)};
+  const int64_t nq256 = (int64_t)((Sq + 255) / 256) * B * H;
+  const int64_t rounds = (nkv + cus - 1) / cus, sweep = (int64_t)((Sq + 63) / 64) * (H / Hk);
+  const bool fits2 = nkv + nq <= cus, fits1 = seg == 1 && nkv + nq256 <= cus;
+  const bool tail = seg == 1 && rounds > 1 && 5 * nkv < 4 * rounds * cus && sweep >= 5 && sweep <= 48;
+  return NcFused{fits2 || fits1 || tail, false, fits2 || (!fits1 && nkv >= 2 * cus)};
+}
+
 // Not causal, D = 64: eight waves, 256 rows a workgroup, one workgroup per CU
 // and round, half the tile DMAs per row.  Pays (1-3 %) on full or nearly full
 // rounds of long sweeps whose rows it does not pad further; elsewhere the
@@ -447,7 +488,10 @@ int launch_dkdv(const fa::BwdArgs &a, hipStream_t stream) {
   if constexpr (D == 64 && CAUSAL) {
     if (a.split_kt > 0) return launch_dkdv_split<E, D, CAUSAL, 2>(a, stream);
   }
-  return dkdv_split2(D, CAUSAL, a.Sk, (int64_t)a.B * a.Hk * a.seg_n)
+  // (the fused launch's layouts where fa_bwd takes it: the same bits)
+  const NcFused nc = nc_fused(a.B, a.Sq, a.Sk, a.H, a.Hk, D, a.seg_n);
+  return (!CAUSAL && nc.on ? nc.kv2
+                           : dkdv_split2(D, CAUSAL, a.Sk, (int64_t)a.B * a.Hk * a.seg_n))
              ? launch_dkdv_split<E, D, CAUSAL, 2>(a, stream)
              : launch_dkdv_split<E, D, CAUSAL, 1>(a, stream);
 }
@@ -455,7 +499,8 @@ int launch_dkdv(const fa::BwdArgs &a, hipStream_t stream) {
 template <typename E, int D, bool CAUSAL>
 int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
   const int64_t heads = (int64_t)a.B * a.H;
-  const bool split = dq_split2(D, CAUSAL, a.Sq, heads);
+  const NcFused nc = nc_fused(a.B, a.Sq, a.Sk, a.H, a.Hk, D, 1);
+  const bool split = !CAUSAL && nc.on ? nc.q2 : dq_split2(D, CAUSAL, a.Sq, heads);
   // Eight waves sharing each K / V tile, as in the forward: D = 64 (256
   // queries, no key split) below two rounds ((1,4096,16) 235.7 us the
   // backward, 238.2 with four waves, (1,4096,30) 466 / 494, (1,4096,32) 466 /
@@ -490,7 +535,7 @@ int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
                : launch_dq_split<E, D, CAUSAL, 1, false>(a, stream);
 }
 
-// Fused causal backward (fa::fa_bwd_fused_kernel; bwd_fused decides): the pre-pass,
+// Fused backward (fa::fa_bwd_fused_kernel; bwd_fused decides): the pre-pass,
 // which computes delta and zeroes the key-block split's counters, then
 // one launch of every dK/dV block followed by every dQ block.
 struct FusedBwd {
@@ -533,20 +578,28 @@ int launch_bwd_fused_as(FusedBwd f, hipStream_t stream) {
 
 template <typename E, int D, bool CAUSAL>
 int launch_bwd_fused(const FusedBwd &f, hipStream_t stream) {
-  if constexpr (D <= 64 && CAUSAL) {
+  if constexpr (D <= 64) {
     if (f.kv_split2)
       return f.q_split2 ? launch_bwd_fused_as<E, D, CAUSAL, 2, 2>(f, stream)
                         : launch_bwd_fused_as<E, D, CAUSAL, 2, 1>(f, stream);
     return f.q_split2 ? launch_bwd_fused_as<E, D, CAUSAL, 1, 2>(f, stream)
                       : launch_bwd_fused_as<E, D, CAUSAL, 1, 1>(f, stream);
-  } else if constexpr (D == 128 && CAUSAL) {
+  } else {
     // the eight-wave dK/dV layout beside eight-wave dQ blocks
     return f.q_split2 ? launch_bwd_fused_as<E, D, CAUSAL, 1, 2>(f, stream)
                       : launch_bwd_fused_as<E, D, CAUSAL, 1, 1>(f, stream);
+  }
+}
+
+// The fused launch's layouts.
+void fused_layouts(FusedBwd &f, const Shape &s, int causal, int seg_n) {
+  if (causal) {
+    f.kv_split2 = dkdv_split2(s.D, true, s.Sk, (int64_t)s.B * s.Hk * seg_n);
+    f.q_split2 = dq_split2(s.D, true, s.Sq, (int64_t)s.B * s.H);
   } else {
-    (void)f;
-    (void)stream;
-    return FA_ERR_HEAD_DIM;   // run_bwd picks the fused path for causal grids only
+    const NcFused nc = nc_fused(s.B, s.Sq, s.Sk, s.H, s.Hk, s.D, seg_n);
+    f.kv_split2 = nc.kv2;
+    f.q_split2 = nc.q2;
   }
 }
 
@@ -1157,7 +1210,8 @@ DqSplit dq_split_plan(const Shape &s, int causal) {
   return p;
 }
 
-// The fused backward launch (fa::fa_bwd_fused_kernel) runs the causal
+// The fused backward launch (fa::fa_bwd_fused_kernel) runs the non-causal
+// backwards that nc_fused names, and the causal
 // backwards without the dQ split (whose halves the dK/dV kernel adds after
 // the dQ kernel), unsplit: every D = 32 / 64 one, and the D = 128 ones
 // whose eight-wave dK/dV grid is at most four rounds.  `qplan` is the dQ
@@ -1177,7 +1231,8 @@ DqSplit dq_split_plan(const Shape &s, int causal) {
 //   sweeps leave idle, as the split's second workgroups did, without its
 //   partials.
 bool bwd_fused(const Shape &s, int causal, const DqSplit &qplan, int seg_n = 1) {
-  if (!causal || qplan.split != 0) return false;
+  if (!causal) return nc_fused(s.B, s.Sq, s.Sk, s.H, s.Hk, s.D, seg_n).on;
+  if (qplan.split != 0) return false;
   if (s.D <= 64) return true;
   using T = fa::DkdvTile<128, 1>;
   const int64_t blocks = (s.Sk + T::BK - 1) / T::BK * ((int64_t)s.B * s.Hk) * seg_n;
@@ -1481,8 +1536,7 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
     f.with_pre = true;
     f.akv.seg_n = seg_n;
     f.akv.seg_part = seg_part;
-    f.kv_split2 = plan.split_kt > 0 || dkdv_split2(s.D, true, s.Sk, (int64_t)s.B * s.Hk * seg_n);
-    f.q_split2 = dq_split2(s.D, true, s.Sq, (int64_t)s.B * s.H);
+    fused_layouts(f, s, causal, seg_n);
     hipStream_t st = static_cast<hipStream_t>(stream);
     FA_DISPATCH(launch_bwd_fused, s, causal, f, st);
   }
@@ -1531,8 +1585,7 @@ int run_bwd_blocks(const void *dout, const void *q, const void *k, const void *v
                     nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, &f.aq)))
     return rc;
   f.with_pre = false;
-  f.kv_split2 = dkdv_split2(s.D, true, s.Sk, (int64_t)s.B * s.Hk);
-  f.q_split2 = dq_split2(s.D, true, s.Sq, (int64_t)s.B * s.H);
+  fused_layouts(f, s, causal, 1);
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_bwd_fused, s, causal, f, st);
 }

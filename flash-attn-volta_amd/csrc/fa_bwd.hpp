@@ -13,14 +13,18 @@
 // and delta = rowsum(dO * O) in fp32 (the torch op at :650).  fa_bwd runs
 // them as
 //   causal, D <= 64, and causal D = 128 on grids of at most four rounds
-//   without the dQ split:
+//   without the dQ split; not causal, where the two kernels below would leave
+//   compute units idle (fa_api.hip, nc_fused):
 //                    fa_bwd_preprocess_kernel (delta), then ONE launch of
 //                    fa_bwd_fused_kernel, every dK/dV block and then every
-//                    dQ block in one grid: the dQ blocks fill the slots the
-//                    causal sweeps of unequal length leave idle;
+//                    dQ block in one grid: the dQ blocks fill the slots that
+//                    causal sweeps of unequal length, or a last round, leave
+//                    idle;
 //   otherwise:       fa_bwd_dq_kernel, whose blocks also compute delta from
 //                    the rows their lanes hold and write it, then
 //                    fa_bwd_dkdv_kernel.
+// Where key/value heads are few, the dK/dV blocks run in sweep segments
+// (BwdArgs::seg_n) and fa_bwd_seg_sum_kernel follows.
 // Both ways compute delta with the same fp32 operations in the same order,
 // so the gradients are the same bits.  The standalone entry points
 // fa_bwd_preprocess / fa_bwd_dq / fa_bwd_dkdv run fa_bwd_preprocess_kernel
@@ -1499,12 +1503,12 @@ void fa_bwd_dq_kernel(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Fused backward (causal; four-wave blocks at D <= 64, the eight-wave dK/dV
+// Fused backward (four-wave blocks at D <= 64, the eight-wave dK/dV
 // layout with eight-wave dQ blocks at D = 128): the dK/dV blocks and the dQ blocks of
 // one backward in one grid -- workgroups [0, n_kv) run dkdv_block with
 // `akv`, the rest dq_block with `aq` -- so that the dQ blocks, dispatched
-// after every dK/dV block, fill the slots the causal sweeps of unequal
-// length leave idle, and no kernel boundary drains the GPU between the
+// after every dK/dV block, fill the slots that causal sweeps of unequal
+// length, or a last round that is not full, leave idle, and no kernel boundary drains the GPU between the
 // two.  Both read only the inputs, delta and the row-group maxima (the
 // pre-pass computes them and zeroes the key-block split's counters first)
 // and write disjoint outputs,

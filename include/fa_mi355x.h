@@ -255,13 +255,18 @@ size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, 
  * given the forward's `lse`. Two launches. Causal with D = 32 or 64, and
  * causal D = 128 on grids of at most four workgroups of eight waves per
  * compute unit, in both cases without the dQ query-block split (see
- * fa_bwd_gqa_workspace_bytes) and unsplit:
+ * fa_bwd_gqa_workspace_bytes) and unsplit, and without a mask wherever the
+ * two kernels below would leave compute units idle (most D = 32 / 64 grids;
+ * D = 128 grids that fit the compute units at once or end on a mostly empty
+ * round):
  * fa_bwd_preprocess's kernel (delta = rowsum(o * dout) and the row-group
  * maxima into the workspace), then one launch running every dK/dV
  * workgroup (one per key block, or two for the longest blocks when the
  * workspace has room: fa_bwd_gqa_workspace_bytes) and then every dQ
  * workgroup (one per query block). Otherwise: the dQ kernel, which also
  * computes delta and the maxima into the workspace, then the dK/dV kernel.
+ * With room for sweep segments (fa_bwd_best_workspace_bytes) a key block is
+ * several workgroups and a third launch adds their fp32 rows.
  * dS is rounded to fp16 for the MFMAs at a power-of-two scale per key,
  * settled per 32- to 128-query tile from the bound |dS| <= max|do| *
  * ||v_key||_1 + max|delta| over the tile's rows (so no scaled dS can
