@@ -387,6 +387,21 @@ int launch_fwd_mode(const fa::FwdArgs &a, hipStream_t stream) {
   return launch_fwd_split<E, D, CAUSAL, KSPLIT, false, NW>(a, stream);
 }
 
+// The forward at D = 128 without a key split in eight waves, 256 rows a
+// workgroup (half the tile DMAs per row, one workgroup per CU): long sweeps
+// whose rows it does not pad further, not causal on full rounds only.
+// Measured, four waves -> eight: not causal (1,4096,16) 139 -> 134 us,
+// (1,4096,32) 272 -> 264, (4,4096,16) 518 -> 507, (2,8192,16) 1012 -> 983, but
+// (1,4096,20) 205 -> 223, (1,4096,28) 252 -> 258, (4,1024,32) 85 -> 86; causal
+// (1,16384,16) 1008 -> 981, (1,8192,32/8) 494 -> 479, (1,8192,16) 277 -> 273, but
+// (1,9000,20) 447 -> 456, (1,7000,32/8) 390 -> 398 (an odd count of 128-row
+// blocks), (4,4096,16) 284 -> 286, (2,2048,32) 86 -> 93.
+bool eight_waves_128(bool causal, int Sq, int Sk, int64_t heads) {
+  const int64_t n = (int64_t)((Sq + 255) / 256) * heads, cus = device_cus();
+  if (2 * n != grid128(Sq, heads)) return false;
+  return causal ? Sq >= 8192 && n >= cus : n % cus == 0 && Sk >= 2048;
+}
+
 template <typename E, int D, bool CAUSAL>
 int launch_fwd(const fa::FwdArgs &a, hipStream_t stream) {
   const int64_t heads = (int64_t)a.B * a.H;
@@ -410,6 +425,10 @@ int launch_fwd(const fa::FwdArgs &a, hipStream_t stream) {
     // each), long sweeps: (1,4096,8) 69 us, 72 unsplit; (1,4608,8) 131 / 109
     if (grid128(a.Sq, heads) == device_cus() && a.Sk >= 2048)
       return launch_fwd_mode<E, D, CAUSAL, 2, 8>(a, stream);
+  }
+  if constexpr (D == 128) {
+    if (!fwd_split2(D, CAUSAL, a.Sq, heads) && eight_waves_128(CAUSAL, a.Sq, a.Sk, heads))
+      return launch_fwd_mode<E, D, CAUSAL, 1, 8>(a, stream);
   }
   return fwd_split2(D, CAUSAL, a.Sq, heads) ? launch_fwd_mode<E, D, CAUSAL, 2>(a, stream)
                                             : launch_fwd_mode<E, D, CAUSAL, 1>(a, stream);
