@@ -12,7 +12,7 @@ the forward and the node are recorded in C++, and the backward runs on the
 autograd engine's thread without taking the GIL, which a Python backward
 node must take while the thread that called backward() waits for it.  The
 Python Function below is the path for everything else (general layouts,
-D = 16, functorch transforms, torch.compile tracing, or no _fa_torch
+functorch transforms, torch.compile tracing, or no _fa_torch
 build); it keeps the forward's plan on the context and runs the backward
 plan paired with it.  ``_apply`` skips torch's Python-level
 ``Function.apply`` wrapper when no functorch transform is active (it only

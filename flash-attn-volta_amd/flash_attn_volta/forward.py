@@ -314,7 +314,7 @@ class _FwdPlan:
 
 
 def _forward(q, k, v, causal, sm_scale, want_lse, gqa):
-    """General path: pads D = 16 to 32, copies layouts the kernels cannot
+    """General path: copies (D = 16: padded to 32) layouts the kernels cannot
     read in place, handles empty tensors.  Returns (out, lse or None)."""
     D = q.shape[-1]
     if D not in NATIVE_HEAD_DIMS:
