@@ -704,9 +704,10 @@ SplitPlan splitkv_plan(const Shape &s) {
 //     takes `lone` alone on its CU and grows with the workgroups per CU
 //     from where they fill it; a workgroup's start-up; and for a split the
 //     merge launch and its partials' traffic.  Measured, bf16, plain ->
-//     chosen: (1, Sq, 8448 keys, 32 / 8, 128) Sq = 256 90 -> 52 us, 128 92 ->
-//     32, 32 92 -> 19, 400 of 9000 95 -> 75, 200 of 3000 36 -> 27, (2,64,2000)
-//     28 -> 20; (1,1000,9000,14/2,64) 67 -> 50; against it (1,600,3000,32/8,128)
+//     chosen: (1, Sq, 8448 keys, 32 / 8, 128) Sq = 256 90 -> 48 us, 128 91 ->
+//     33, 32 92 -> 21, 400 of 9000 95 -> 74, 200 of 3000 35 -> 27, 512 of 17000
+//     257 -> 176, 256 of 17000 250 -> 98, (2,64,2000) 28 -> 20;
+//     (1,1000,9000,14/2,64) 67 -> 48; against it (1,600,3000,32/8,128)
 //     44 -> 56, (1,300,2000,28/4,128) 27.5 -> 28.5 and (1,200,1000,32/32,128)
 //     16.0 -> 18.6 in two ranges, which the model leaves plain.
 SplitPlan fwd_split_plan(const Shape &s, int causal) {
@@ -722,14 +723,24 @@ SplitPlan fwd_split_plan(const Shape &s, int causal) {
   // (a causal grid's plain sweeps must be near the full length: at least
   // half of the keys lie before the block)
   if (causal && (int64_t)s.Sk < 2 * (int64_t)s.Sq) return none;
-  const double lone = s.D >= 128 ? 0.65 : 0.47, fill = s.D >= 128 ? 0.9 : 0.75;
-  const double start = 6.0;
+  const double lone = s.D >= 128 ? 0.65 : 0.47, start = 6.0;
   auto sweep_us = [&](int64_t wgs, int64_t tiles) {
-    const double w = fill * (double)wgs / (double)cus;
-    return lone * (w > 1.0 ? w : 1.0) * (double)tiles + start;
+    const double w = (double)wgs / (double)cus;   // workgroups per CU
+    double step = lone;
+    if (s.D >= 128) {
+      if (w > 1.0) step = w <= 2.0 ? 0.65 + 0.45 * sqrt(w - 1.0) : 0.7 * w;
+    } else if (0.75 * w > 1.0) {
+      step = lone * 0.75 * w;
+    }
+    return step * (double)tiles + start;
   };
   const int64_t tiles = (s.Sk + 63) / 64, packed = packed_tiles(s);
-  double best = 0.88 * sweep_us(plain, tiles);
+  // (D = 128, a head's K and V past an XCD's L2: the sweeps of a plain grid
+  // of one workgroup per CU or less, which share them only across a head's
+  // query tiles, drift apart and miss: 0.91 us a step at 17000 keys)
+  const double far =
+      s.D >= 128 && plain <= cus && (double)s.Sk * s.D * 4.0 > 6.0e6 ? 1.4 : 1.0;
+  double best = 0.88 * (far * (sweep_us(plain, tiles) - start) + start);
   int64_t best_n = 0;
   for (int64_t n = 2; n <= 32 && 4 * n <= tiles; ++n) {
     const double rows = (double)s.B * s.H * s.Sq * n;

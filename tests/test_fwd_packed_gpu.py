@@ -37,6 +37,7 @@ CHUNKS = [
     (2, 100, 5003, 14, 2, 64, True, F16, True),
     (1, 65, 4000, 4, 4, 32, False, F16, False),     # equal heads
     (1, 256, 8448, 8, 8, 64, True, BF16, False),
+    (1, 70, 12100, 8, 2, 128, False, BF16, False),  # keys past an XCD's L2
 ]
 
 
