@@ -115,6 +115,26 @@ bool kernel_strides(const Tensor &t, int64_t (&st)[4]) {
   return st[1] <= (INT32_MAX - 2 * t.size(3)) / (2 * 127);
 }
 
+// `t` as the kernels read it, its strides in `st`: itself where the layout and
+// alignment allow, else a contiguous copy.
+Tensor kernel_ready(const Tensor &t, int64_t (&st)[4]) {
+  if (kernel_strides(t, st) && aligned(t)) return t;
+  Tensor c = t.clone(at::MemoryFormat::Contiguous);
+  kernel_strides(c, st);
+  return c;
+}
+
+// What a node saved may come back changed: hooks on saved tensors
+// (torch.autograd.graph) return a tensor of their own, save_on_cpu for one a
+// contiguous copy of any view.  The strides that a backward passes are
+// therefore the returned tensor's; one of another shape, type or device than
+// was saved is refused, as the kernels would read past its end.
+void check_saved(const Tensor &t, at::IntArrayRef sizes, at::ScalarType dtype, at::Device device) {
+  TORCH_CHECK(t.defined() && t.sizes() == sizes && t.scalar_type() == dtype &&
+                  t.device() == device,
+              "flash_attn_volta: a saved tensor came back with another shape, dtype or device");
+}
+
 void check(int rc, const char *where) {
   TORCH_CHECK(rc == FA_OK, where, ": ", fa_strerror(rc), " (status ", rc, ")");
 }
@@ -152,39 +172,45 @@ struct FlashAttnFn : public torch::autograd::Function<FlashAttnFn> {
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const Tensor &q = s[0], &k = s[1], &v = s[2], &out = s[3], &lse = s[4];
     const Plan &p = *reinterpret_cast<const Plan *>(ctx->saved_data["plan"].toInt());
     const bool split = ctx->saved_data["split"].toBool();
-    const c10::DeviceGuard guard(q.device());
+    // the engine hands dO over in out's shape, on its device
+    const at::Device device = grads[0].device();
+    const auto dtype = (p.dtype & ~FA_HALF_COLS) == FA_DTYPE_BF16 ? at::kBFloat16 : at::kHalf;
+    const int64_t cols = grads[0].size(3);
+    const c10::DeviceGuard guard(device);
+    for (int i : {0, 3}) check_saved(s[i], {p.B, p.Sq, p.H, cols}, dtype, device);
+    for (int i : {1, 2}) check_saved(s[i], {p.B, p.Sk, p.Hk, cols}, dtype, device);
+    check_saved(s[4], {p.B, p.H, p.Sq}, at::kFloat, device);
+    int64_t q_st[4], k_st[4], v_st[4], o_st[4], do_st[4];
+    const Tensor q = kernel_ready(s[0], q_st), k = kernel_ready(s[1], k_st),
+                 v = kernel_ready(s[2], v_st), out = kernel_ready(s[3], o_st);
+    const Tensor lse = s[4].is_contiguous() && aligned(s[4])
+                           ? s[4] : s[4].clone(at::MemoryFormat::Contiguous);
     // dO as the kernels read it: the forward's dtype, in place when its
     // layout allows (a model's transposed (B, H, S, D) gradient does: making
     // it contiguous cost 11 us of 113 at (8,1024,12,64)), 16-byte aligned
-    Tensor dout = grads[0];
-    if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
-    int64_t do_st[4];
-    if (!kernel_strides(dout, do_st) || !aligned(dout)) {
-      dout = dout.clone(at::MemoryFormat::Contiguous);
-      std::copy(p.o_st, p.o_st + 4, do_st);
-    }
-    Tensor dq = at::empty({p.B, p.Sq, p.H, q.size(3)}, q.options());
+    const Tensor dout = kernel_ready(
+        grads[0].scalar_type() == dtype ? grads[0] : grads[0].to(dtype), do_st);
+    Tensor dq = at::empty({p.B, p.Sq, p.H, cols}, q.options());
     // separate allocations, as the Python path's
-    Tensor dk = at::empty({p.B, p.Sk, p.Hk, q.size(3)}, q.options());
-    Tensor dv = at::empty({p.B, p.Sk, p.Hk, q.size(3)}, q.options());
+    Tensor dk = at::empty({p.B, p.Sk, p.Hk, cols}, q.options());
+    Tensor dv = at::empty({p.B, p.Sk, p.Hk, cols}, q.options());
     const size_t nb = split ? p.ws_split : p.ws_plain;
     Tensor ws = at::empty({(int64_t)nb}, q.options().dtype(at::kByte));
     void *stream = stream_of(q);
     if (p.gqa) {
       check(fa_bwd_gqa(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                        lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                       ws.data_ptr(), nb, p.B, p.Sq, p.Sk, p.H, p.Hk, p.D, do_st, p.q_st,
-                       p.k_st, p.v_st, p.o_st, p.dq_st, p.dk_st, p.dk_st, p.scale, p.causal,
+                       ws.data_ptr(), nb, p.B, p.Sq, p.Sk, p.H, p.Hk, p.D, do_st, q_st,
+                       k_st, v_st, o_st, p.dq_st, p.dk_st, p.dk_st, p.scale, p.causal,
                        p.dtype, stream),
             "fa_bwd_gqa");
     } else {
       check(fa_bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                    lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                   ws.data_ptr(), nb, p.B, p.Sq, p.H, p.D, do_st, p.q_st, p.k_st, p.v_st,
-                   p.o_st, p.dq_st, p.dk_st, p.dk_st, p.scale, p.causal, stream),
+                   ws.data_ptr(), nb, p.B, p.Sq, p.H, p.D, do_st, q_st, k_st, v_st,
+                   o_st, p.dq_st, p.dk_st, p.dk_st, p.scale, p.causal, stream),
             "fa_bwd");
     }
     return {dq, dk, dv, Tensor(), Tensor()};
@@ -221,6 +247,14 @@ void table_strides(const Tensor &t, int64_t (&st)[2]) {
   st[1] = t.size(d - 2) == 1 ? 0 : t.stride(d - 2);
 }
 
+// A table that the kernels read in place, its strides in `st`: unit D stride,
+// the others non-negative multiples of 8 elements, 16-byte aligned.
+bool table_ready(const Tensor &t, int64_t (&st)[2]) {
+  table_strides(t, st);
+  return t.stride(t.dim() - 1) == 1 && st[0] >= 0 && st[1] >= 0 && st[0] % 8 == 0 &&
+         st[1] % 8 == 0 && aligned(t);
+}
+
 struct RopeFn : public torch::autograd::Function<RopeFn> {
   static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k,
                                const Tensor &cos, const Tensor &sin, const OptTensor &wq,
@@ -247,34 +281,50 @@ struct RopeFn : public torch::autograd::Function<RopeFn> {
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const Tensor &cos = s[2], &sin = s[3], &wq = s[4], &wk = s[5];
     const double eps = ctx->saved_data["eps"].toDouble();
-    const c10::DeviceGuard guard(cos.device());
+    // the engine hands the gradients over in the outputs' shapes and dtype
+    const auto dtype = grads[0].scalar_type();
+    const at::Device device = grads[0].device();
+    const c10::DeviceGuard guard(device);
+    const int B = (int)grads[0].size(0), S = (int)grads[0].size(1), H = (int)grads[0].size(2),
+              Hk = (int)grads[1].size(2), D = (int)grads[0].size(3);
+    const bool norm[2] = {s[4].defined(), s[5].defined()};
+    Tensor cos = s[2], sin = s[3], w[2];
+    const bool one = cos.dim() == 3 && cos.size(0) == 1;
+    check_saved(cos, cos.dim() == 2 ? at::DimVector{S, D} : at::DimVector{one ? 1 : B, S, D}, dtype,
+                device);
+    check_saved(sin, cos.sizes(), dtype, device);
+    int64_t g_st[2][4], x_st[2][4], d_st[2][4], cs[2], sn[2];
+    if (!table_ready(cos, cs) || !table_ready(sin, sn) || cs[0] != sn[0] || cs[1] != sn[1]) {
+      cos = cos.clone(at::MemoryFormat::Contiguous);
+      sin = sin.clone(at::MemoryFormat::Contiguous);
+      table_ready(cos, cs);
+    }
     const auto opt = cos.options();
-    int64_t g_st[2][4], x_st[2][4], d_st[2][4], cs[2];
     Tensor g[2], x[2], d[2], dw[2];
     for (int i = 0; i < 2; ++i) {
-      g[i] = grads[i].scalar_type() == cos.scalar_type() ? grads[i]
-                                                         : grads[i].to(cos.scalar_type());
-      if (!kernel_strides(g[i], g_st[i]) || !aligned(g[i])) {
-        g[i] = g[i].clone(at::MemoryFormat::Contiguous);
-        kernel_strides(g[i], g_st[i]);
+      g[i] = kernel_ready(grads[i].scalar_type() == dtype ? grads[i] : grads[i].to(dtype),
+                          g_st[i]);
+      if (norm[i]) {
+        check_saved(s[i], g[i].sizes(), dtype, device);
+        check_saved(s[4 + i], {D}, dtype, device);
+        x[i] = kernel_ready(s[i], x_st[i]);
+        w[i] = s[4 + i].is_contiguous() && aligned(s[4 + i])
+                   ? s[4 + i] : s[4 + i].clone(at::MemoryFormat::Contiguous);
+        dw[i] = at::empty({D}, opt);   // the weight's dtype
+      } else {
+        x[i] = g[i];   // read for a normed side only
+        std::copy(g_st[i], g_st[i] + 4, x_st[i]);
       }
-      x[i] = s[i].defined() ? s[i] : g[i];   // read for a normed side only
-      kernel_strides(x[i], x_st[i]);
       d[i] = at::empty(g[i].sizes(), opt);
       kernel_strides(d[i], d_st[i]);
-      if (s[4 + i].defined()) dw[i] = at::empty({g[i].size(3)}, opt);   // the weight's dtype
     }
-    table_strides(cos, cs);
-    const int B = (int)g[0].size(0), S = (int)g[0].size(1), H = (int)g[0].size(2),
-              Hk = (int)g[1].size(2), D = (int)g[0].size(3);
     Tensor ws;
-    if (wq.defined() || wk.defined())
+    if (norm[0] || norm[1])
       ws = at::empty({(int64_t)fa_rope_qk_workspace_bytes(B, S, H, Hk, D)}, opt.dtype(at::kByte));
     auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
     check(fa_rope_qk_bwd(g[0].data_ptr(), g[1].data_ptr(), x[0].data_ptr(), x[1].data_ptr(),
-                         cos.data_ptr(), sin.data_ptr(), ptr(wq), ptr(wk), (float)eps,
+                         cos.data_ptr(), sin.data_ptr(), ptr(w[0]), ptr(w[1]), (float)eps,
                          d[0].data_ptr(), d[1].data_ptr(), static_cast<float *>(ptr(dw[0])),   // FA_DW_16
                          static_cast<float *>(ptr(dw[1])), ptr(ws),
                          ws.defined() ? (size_t)ws.numel() : 0, B, S, H, Hk, D, g_st[0], g_st[1],
@@ -307,19 +357,14 @@ std::optional<std::tuple<Tensor, Tensor>> rope(const Tensor &q, const Tensor &k,
   int64_t st[4];
   if (!same(q) || !same(k) || !kernel_strides(q, st) || !kernel_strides(k, st))
     return std::nullopt;
+  int64_t c_st[2], s_st[2];
   for (const Tensor *t : {&cos, &sin}) {
     const int64_t d = t->dim();
     if ((d != 2 && d != 3) || t->size(d - 1) != D || t->size(d - 2) != S ||
         (d == 3 && t->size(0) != 1 && t->size(0) != B) || !same(*t) || t->requires_grad() ||
-        t->stride(d - 1) != 1)
+        !table_ready(*t, t == &cos ? c_st : s_st))
       return std::nullopt;
-    int64_t ts[2];
-    table_strides(*t, ts);
-    if (ts[0] < 0 || ts[1] < 0 || ts[0] % 8 != 0 || ts[1] % 8 != 0) return std::nullopt;
   }
-  int64_t c_st[2], s_st[2];
-  table_strides(cos, c_st);
-  table_strides(sin, s_st);
   if (cos.sizes() != sin.sizes() || c_st[0] != s_st[0] || c_st[1] != s_st[1]) return std::nullopt;
   for (const OptTensor *w : {&wq, &wk}) {
     if (!*w) continue;

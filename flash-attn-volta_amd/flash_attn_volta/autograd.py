@@ -43,7 +43,10 @@ def _saved_backward(ctx, do, gqa):
     if not do.is_contiguous():
         do = do.contiguous()
     plan = ctx.plan
-    if plan is not None:
+    # a hook on saved tensors may hand back other layouts than were saved
+    if lse.data_ptr() % 16:
+        lse = lse.clone()
+    if plan is not None and plan.reads(q, k, v, out, lse):
         bwd = plan.bwd if plan.bwd is not None else plan.make_bwd()
         r = bwd(do, q, k, v, out, lse)
         if r is not None:

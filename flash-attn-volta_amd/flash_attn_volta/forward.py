@@ -217,7 +217,7 @@ class _FwdPlan:
     results."""
     __slots__ = ("fn", "name", "args", "out_shape", "lse_shape", "dtype", "code", "device", "idx",
                  "like", "ws_bytes", "causal", "sm_scale", "gqa", "sizes", "st", "q_stride",
-                 "k_stride", "bwd", "cpp")
+                 "k_stride", "v_stride", "k_shape", "bwd", "cpp")
 
     @classmethod
     def build(cls, q, k, v, causal, sm_scale, want_lse, gqa):
@@ -238,6 +238,7 @@ class _FwdPlan:
         p.like = q.stride() == o_st          # empty_like(q) is then contiguous
         st = (kernel_strides(q), kernel_strides(k), kernel_strides(v), _strides_c(p.out_shape, o_st))
         p.sizes, p.st, p.q_stride, p.k_stride = (B, Sq, Sk, H, Hk, D), st, q.stride(), k.stride()
+        p.v_stride, p.k_shape = v.stride(), k.shape
         p.bwd = None
         p.cpp = 0
         # the schedule with a workspace (split-KV for decode shapes, the
@@ -275,6 +276,16 @@ class _FwdPlan:
         if rc:
             _capi.check(rc, self.name)
         return out, lse
+
+    def reads(self, q, k, v, out, lse) -> bool:
+        """Tensors laid out as this plan's q, k, v, out and LSE."""
+        return (q.stride() == self.q_stride and k.stride() == self.k_stride
+                and v.stride() == self.v_stride and out.is_contiguous() and lse.is_contiguous()
+                and q.shape == out.shape == self.out_shape and k.shape == v.shape == self.k_shape
+                and lse.shape == self.lse_shape
+                and q.dtype == k.dtype == v.dtype == out.dtype == self.dtype
+                and lse.dtype == torch.float32
+                and q.device == k.device == v.device == out.device == lse.device == self.device)
 
     def make_bwd(self):
         """The backward plan paired with this forward (autograd.py): its
