@@ -1301,9 +1301,11 @@ size_t segment_bytes(const Shape &s) {
 // head of its group, so few key/value heads leave few, long workgroups:
 // (1, 4000, 28 heads / 4, 128) causal is 128 workgroups of up to 441 query
 // tiles on 256 CUs.  A segment costs its fp32 rows (written once, read once
-// by the sum) and a workgroup's start-up, so as few as fill the GPU.
-// Measured, the backward (1 segment -> chosen), causal, D = 128:
-//   (1,4000,28/4) 762 -> 444 us (2; 4: 444, 8: 469), (1,3000,28/4) 563 -> 272
+// by the sum) and a workgroup's start-up, so as few as fill the GPU: never
+// on grids of more than one round, never more than two rounds of segments,
+// which bounds their rows by 64 MiB.
+// Measured, the backward, us (1 segment -> chosen), causal, D = 128:
+//   (1,4000,28/4) 762 -> 444 (2; 4: 444, 8: 469), (1,3000,28/4) 563 -> 272
 //   (3), (1,2048,16/2) 428 -> 91 (8), (1,1024,32/8) 121 -> 62 (3), (1,700,64/8)
 //   162 -> 65 (4; 6: 72), (1,512,32/8) 67 -> 35 (4; 6: 40), (1,300,28/4) 72 -> 31
 //   (8), (1,128,28/4) 37 -> 24 (7), (1,3500,32/8) 411 -> 388 (2), (1,4096,32/8)
@@ -1312,29 +1314,53 @@ size_t segment_bytes(const Shape &s) {
 // D = 64: (1,4096,14/2) 396 -> 134 (8), (1,3000,14/2) 300 -> 80 (8; 11: 89),
 //   (1,2048,32/8) 131 -> 84 (3), (1,700,14/2) 78 -> 24 (13);
 // equal heads: (1,2048,4/4) 65 -> 55, (2,1500,4/4) 54 -> 48 (2), but
-//   (1,2048,8/8) +6 %;
-// not causal: (1,2048,32/4,128) 467 -> 254 (4), (1,3000,32/8,128) 754 -> 529
-//   (4), (1,4096,4/4,128) 161 -> 149 (2), (1,4096,14/2,64) 470 -> 245 (8), but
-//   (2,1024,8/8,64) (16-tile sweeps) +24 % with 2.
+//   (1,2048,8/8) +6 %.
+// Not causal, beside the fused launch (f; the two kernels otherwise),
+// D = 128: (1,2048,32/4) f 434 -> 255 (4), (1,3500,8/2) f 367 -> 208 (4; 9:
+//   219), (1,2048,16/2) f 408 -> 141 (8), (1,1024,32/8) f 118 -> 86 (4),
+//   (1,1500,64/8) f 367 -> 302 (2; 8: 311), (1,2560,32/8) f 431 -> 413 (3), but
+//   (1,2200,32/8) f 302 / 355 (3), (1,3000,32/8) f 520 / 549 (4), (1,8300,32/8)
+//   f 3820 / 4028 (6);
+// D = 64, fused: (1,4096,14/2) 409 -> 231 (8), (1,2048,8/2) 114 -> 50 (8),
+//   (1,5000,16/4) 468 -> 397 (3), (1,4096,2/2) 61 -> 58 (4), (1,4096,40/10) 649 ->
+//   599 (3), but (1,4096,4/4) 77 / 80 (4), (1,3000,6/6) 72 / 78 (2),
+//   (1,6000,12/12) 394 / 448 (5).
+// Equal heads at D = 128 whose dK/dV and dQ blocks all have a CU of their
+// own (the fused launch's own condition on one round) only as far as they
+// keep it: (1,4096,2/2) f 114 -> f 99 (3; 4, two kernels: 111), (1,2048,4/4) f
+// 63 -> f 59 (2), (1,4096,4/4) f 138 / 150 (2), (1,4096,5/5) f 165 / 210 (3).
 int dkdv_segments(const Shape &s, int causal) {
   const int64_t grp = s.H / s.Hk;
-  const int64_t blocks = (int64_t)((s.Sk + 127) / 128) * s.B * s.Hk;
-  const int64_t slots = (s.D >= 128 ? 1 : 2) * (int64_t)device_cus();
+  const int64_t blocks = (int64_t)((s.Sk + 127) / 128) * s.B * s.Hk, cus = device_cus();
+  const int64_t slots = (s.D >= 128 ? 1 : 2) * cus;
+  if (blocks > slots) return 1;
   const int64_t sweep = causal ? causal_tiles(s, 0, 128, 64) : (int64_t)((s.Sq + 63) / 64) * grp;
   if (!causal) {
-    // rounds times (tiles of a segment + 3, a workgroup's start-up), at
-    // least 16 tiles each; 10 % better at least
-    int64_t best = 1, cost = (blocks + slots - 1) / slots * (sweep + 3) * 9 / 10;
-    for (int64_t n = 2; n <= 16 && 16 * n <= sweep; ++n) {
-      const int64_t c = (blocks * n + slots - 1) / slots * ((sweep + n - 1) / n + 3);
+    // rounds times (tiles of a segment + 3, a workgroup's start-up), in
+    // query tiles of about `tile` us, plus the rows' write and read at 4
+    // TB/s; at least 16 tiles each; 10 % better at least than whole sweeps.
+    // (D <= 64 grids of at most half a round run the query-split blocks,
+    // which halve a whole sweep at some 15 % more work.)
+    const NcFused whole = nc_fused(s.B, s.Sq, s.Sk, s.H, s.Hk, s.D, 1);
+    const double tile = s.D >= 128 ? 1.2 : (s.D == 64 ? 0.6 : 0.4);
+    const double rows = 2.0 * (double)segment_bytes(s) / 4.0e6 / tile;
+    const bool halves = s.D <= 64 && whole.kv2 && 2 * blocks <= slots;
+    double cost = halves ? 0.575 * (double)sweep + 3.0 : 0.9 * ((double)sweep + 3.0);
+    int64_t most = 2 * slots / blocks;
+    if (s.D >= 128 && grp == 1 && whole.on)
+      most = (cus - grid128(s.Sq, (int64_t)s.B * s.H)) / blocks;
+    int best = 1;
+    for (int64_t n = 2; n <= 16 && n <= most && 16 * n <= sweep; ++n) {
+      const int64_t rounds = (blocks * n + slots - 1) / slots;
+      const double c =
+          (double)(rounds * ((sweep + n - 1) / n + 3)) + rows * (double)n;
       if (c < cost) {
-        best = n;
+        best = (int)n;
         cost = c;
       }
     }
-    return (int)best;
+    return best;
   }
-  if (blocks > slots) return 1;
   if (grp == 1) {
     if (s.D != 128 || 8 * blocks > 3 * slots || sweep < 20) return 1;
     DkdvSplit plan;

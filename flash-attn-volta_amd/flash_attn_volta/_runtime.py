@@ -98,8 +98,8 @@ def convert(name: str, first: int, values) -> tuple:
 # into a graph gets a fresh tensor instead: the graph keeps the addresses it
 # recorded, which a later growth here would free.  At most
 # MAX_CACHED_STREAMS streams keep one (least recently used dropped first),
-# so threads drawing streams from a pool cannot pin a workspace each (up to
-# ~64 MiB for the split schedule of a small causal grid); the memory of a
+# so threads drawing streams from a pool cannot pin a workspace each (delta
+# and up to 80 MiB of partials); the memory of a
 # dropped one goes back to torch's caching allocator.
 MAX_CACHED_STREAMS = 4
 _WS: "collections.OrderedDict" = collections.OrderedDict()

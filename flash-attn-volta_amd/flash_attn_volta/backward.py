@@ -196,7 +196,7 @@ def _backward(do, q, k, v, o, lse, causal, sm_scale, gqa):
 # their split schedule (longest key / query blocks swept by two workgroups;
 # 8-20 % faster on those grids, at up to 80 MiB of fp32 partials) and grids
 # of few key blocks sweep each in segments (grouped heads: up to 5 times
-# faster, at segments x 8 bytes per element of K); set it
+# faster, at segments x 8 bytes per element of K, at most 64 MiB); set it
 # to False to cap the workspace at delta's B * H * Sq * 4 bytes (the
 # unsplit schedule, same results to rounding).  The workspace is cached per
 # stream and reused by later calls (_runtime.workspace;

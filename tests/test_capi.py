@@ -177,6 +177,36 @@ def test_split_workspace_bytes(lib):
     assert lib.fa_bwd_gqa_workspace_bytes(1, 700, 1000, 8, 2, 96, 1) == 0        # bad D
 
 
+def test_best_workspace_is_bounded(lib):
+    """fa_bwd_best_workspace_bytes over a sweep of sizes: the minimum plus at
+    most the splits' 80 MiB and 4 KiB, or whole segments of at most 64 MiB;
+    nothing beyond fa_bwd_gqa_workspace_bytes on grids of more than a round of
+    128-key blocks (one per CU at D = 128, two below; 256 CUs without a GPU)."""
+    seen = set()
+    for B in (1, 2, 3, 4):
+        for S in (64, 300, 1000, 2200, 3000, 4096, 4200, 6000, 8300, 11200, 13823, 32768):
+            for H, Hk in ((1, 1), (4, 4), (12, 12), (32, 8), (64, 8), (28, 4), (32, 4), (8, 1)):
+                for D in (32, 64, 128):
+                    for causal in (0, 1):
+                        best = lib.fa_bwd_best_workspace_bytes(B, S, S, H, Hk, D, causal)
+                        gqa = lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, Hk, D, causal)
+                        mini = lib.fa_bwd_workspace_bytes(B, S, H, D)
+                        assert mini <= gqa <= mini + (80 << 20) + 4096
+                        one = 2 * B * Hk * S * D * 4
+                        blocks = (S + 127) // 128 * B * Hk
+                        if best == gqa:
+                            continue
+                        n, rest = divmod(best - mini, one)
+                        assert rest == 0 and 2 <= n <= 16 and n * one <= 64 << 20
+                        assert blocks <= (256 if D == 128 else 512)
+                        seen.add((D, causal, n))
+    assert len(seen) > 20
+    # the fused launch's own grids run whole sweeps
+    for B, S, H in ((1, 3000, 12), (1, 4096, 4), (1, 1500, 8), (2, 1000, 10), (4, 1500, 6)):
+        assert lib.fa_bwd_best_workspace_bytes(B, S, S, H, H, 128, 0) == \
+            lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, H, 128, 0)
+
+
 def test_bwd_validation(lib):
     assert _bwd(lib, ws=None) == _capi.FA_ERR_WORKSPACE
     assert _bwd(lib, ws_bytes=16) == _capi.FA_ERR_WORKSPACE
