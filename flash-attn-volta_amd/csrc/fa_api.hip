@@ -281,14 +281,28 @@ bool dkdv_split2(int D, bool causal, int Sk, int64_t heads) {
 //     0.75 on sweeps of 8 tiles or more ((1,4096,4) 105 / 86, (4,512,12) 25 / 23,
 //     (4,1000,8) 41 / 45), both for single 64-row blocks.
 //   D = 32 (the same lines): (2,1000,25) 57 -> 42, (1,4096,16) 163 -> 145.
-//   D = 128, one eight-wave workgroup per CU: where every block has a CU of
-//     its own at once ((1,700,12) 42 -> 33, (1,2048,4) 77 -> 58, (1,1500,8) 73 ->
-//     54, (2,1000,10) 69 -> 53), or the dK/dV grid's last round is mostly empty
-//     and the sweeps are of 5 to 48 tiles ((4,1500,6) 166 -> 121, (1,3000,12)
-//     283 -> 239, (2,3000,12) 486 -> 421, (8,300,12) 57 -> 48); against it
-//     (1,4096,20) 668 / 687, (1,6000,12) 924 / 945, (16,512,12) 147 / 158,
-//     (20,197,12) 62 / 64, and in segments (1,3000,4) 105 / 118, (1,3000,32/8)
-//     537 / 554.
+//   D = 128, one eight-wave workgroup per CU (whole sweeps on both sides):
+//     where every block has a CU of its own at once ((1,700,12) 42 -> 33,
+//     (1,2048,4) 86 -> 63, (1,1500,8) 73 -> 54, (2,1000,10) 69 -> 53);
+//     grouped heads on up to three quarters of a round ((1,3000,32/8) 561 ->
+//     520, (1,2200,32/8) 392 -> 302, (3,1024,32/8) 210 -> 200, (1,4096,24/6) 732 ->
+//     695; on more of it (1,4096,28/7) 834 / 851, equal heads (1,4096,6) 213 /
+//     274);
+//     where the dK/dV grid's last round is mostly empty.  Up to 0.8 of its
+//     rounds on sweeps of 5 to 48 tiles ((4,1500,6) 166 -> 121, (1,3000,12) 299 ->
+//     222, (2,3000,12) 486 -> 421, (8,300,12) 56 -> 47; against it (16,512,12)
+//     147 / 158, (20,197,12) 62 / 64, (6,1024,8) 127 / 133, (10,1024,8) 201 / 198)
+//     and of grouped heads up to 64 tiles or on two rounds ((1,4096,36/9) 1364 ->
+//     1045, (1,4096,48/12) 1492 -> 1394, (5,1024,32/8) 383 -> 340, (9,1024,32/8)
+//     636 / 638; (10,1024,32/8) 677 / 721); longer sweeps
+//     up to 0.65 of two rounds ((1,4096,9) 393 -> 289, (1,4096,10) 399 -> 306;
+//     (1,4096,11) 406 / 422) and 0.85 of three and more ((1,4096,17) 649 -> 566,
+//     (1,4096,20) 656 -> 615, (1,6000,12) 940 -> 802, (1,11200,12) 2888 -> 2682,
+//     (1,4096,33) 1111 -> 1058, (1,8300,32/8) 4623 -> 3820, (2,4200,32/8) 2340 ->
+//     1996, (4,4100,64/8) 8788 -> 8298, (3,13823,32/4) 34250 -> 32290;
+//     (1,4096,22) 670 / 696, (1,4096,24) 704 / 720).
+//     With segments only where every block has a CU ((2,1024,32/8), 2: 83, two
+//     kernels 96; (1,3500,8/2), 4: 246 / 207).
 struct NcFused {
   bool on, kv2, q2;   // kv2, q2: the two-halves layouts of dK/dV and dQ
 };
@@ -302,8 +316,13 @@ NcFused nc_fused(int B, int Sq, int Sk, int H, int Hk, int D, int seg) {
   const int64_t nq256 = (int64_t)((Sq + 255) / 256) * B * H;
   const int64_t rounds = (nkv + cus - 1) / cus, sweep = (int64_t)((Sq + 63) / 64) * (H / Hk);
   const bool fits2 = nkv + nq <= cus, fits1 = seg == 1 && nkv + nq256 <= cus;
-  const bool tail = seg == 1 && rounds > 1 && 5 * nkv < 4 * rounds * cus && sweep >= 5 && sweep <= 48;
-  return NcFused{fits2 || fits1 || tail, false, fits2 || (!fits1 && nkv >= 2 * cus)};
+  const bool grouped = H > Hk, few = seg == 1 && grouped && 4 * nkv <= 3 * cus;
+  // the last round mostly empty: nkv under `full` percent of its rounds
+  const int full = sweep <= 48 || (grouped && (sweep <= 64 || rounds == 2)) ? 80
+                   : rounds == 2                                            ? 65
+                                                                            : 85;
+  const bool tail = seg == 1 && rounds > 1 && sweep >= 5 && 100 * nkv < full * rounds * cus;
+  return NcFused{fits2 || fits1 || few || tail, false, fits2 || (!fits1 && nkv >= 2 * cus)};
 }
 
 // Not causal, D = 64: eight waves, 256 rows a workgroup, one workgroup per CU

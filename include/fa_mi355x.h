@@ -257,8 +257,8 @@ size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, 
  * compute unit, in both cases without the dQ query-block split (see
  * fa_bwd_gqa_workspace_bytes) and unsplit, and without a mask wherever the
  * two kernels below would leave compute units idle (most D = 32 / 64 grids;
- * D = 128 grids that fit the compute units at once or end on a mostly empty
- * round):
+ * D = 128 grids that fit the compute units at once, are grouped heads on part
+ * of a round, or end on a mostly empty round):
  * fa_bwd_preprocess's kernel (delta = rowsum(o * dout) and the row-group
  * maxima into the workspace), then one launch running every dK/dV
  * workgroup (one per key block, or two for the longest blocks when the

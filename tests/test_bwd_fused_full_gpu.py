@@ -32,6 +32,10 @@ SQUARE = [
     (8, 301, 12, 128),                                 # a mostly empty last round
     (1, 2048, 16, 128),                                # a full round: two kernels
     (16, 197, 12, 128),                                # sweeps under 5 tiles: two kernels
+    (1, 3200, 11, 128),                                # 50-tile sweeps, 275 blocks of 512
+    (1, 3200, 14, 128),                                # 350 of 512: two kernels
+    (1, 3200, 24, 128),                                # 600 of 768
+    (1, 3200, 26, 128),                                # 650 of 768: two kernels
 ]
 
 
@@ -56,12 +60,15 @@ CASES = [
     (2, 600, 600, 6, 2, 64, BF16), (4, 500, 333, 12, 12, 64, F16), (1, 1024, 1024, 4, 4, 64, F16),
     (2, 150, 400, 8, 4, 32, BF16), (1, 1500, 700, 4, 4, 128, F16), (2, 333, 1000, 10, 10, 128, BF16),
     (8, 301, 301, 12, 12, 128, F16), (1, 500, 500, 14, 2, 128, BF16),
+    (2, 200, 3000, 12, 4, 128, BF16),                  # grouped heads, three quarters of a round
+    (2, 200, 3100, 12, 4, 128, F16),                   # more of it: two kernels
+    (1, 130, 4600, 64, 8, 128, F16),                   # grouped heads, 288 blocks of 512
 ]
 
 
 @pytest.mark.parametrize("case", CASES, ids=["x".join(str(x) for x in c[:6]) for c in CASES])
 def test_fused_full_matches_oracle(case):
-    from flash_attn_volta import flash_attn_backward_gqa, flash_attn_forward_gqa
+    from flash_attn_volta import _capi, flash_attn_backward_gqa, flash_attn_forward_gqa
     B, Sq, Sk, H, Hk, D, dtype = case
     print(f"[case] fused full vs oracle {case}", flush=True)
     q, k, v, do = orc.make_inputs_gqa(B, Sq, Sk, H, Hk, D, seed=28, dtype=dtype)
@@ -72,7 +79,10 @@ def test_fused_full_matches_oracle(case):
     o, lse = flash_attn_forward_gqa(qd, kd, vd, return_softmax_lse=True)
     got = flash_attn_backward_gqa(dod, qd, kd, vd, o, lse)
     again = flash_attn_backward_gqa(dod, qd, kd, vd, o, lse)
+    least = _bwd_capi(dod, qd, kd, vd, o, lse, False,
+                      _capi.load().fa_bwd_workspace_bytes(B, Sq, H, D), 0xFF)
     tol = TOL if dtype == F16 else 4e-2
-    for name, a, b, r in zip(("dq", "dk", "dv"), got, again, ref):
+    for name, a, b, c, r in zip(("dq", "dk", "dv"), got, again, least, ref):
         assert max_abs(a, r) < tol, name
         assert torch.equal(a, b), name
+        assert max_abs(c, r) < tol, name
