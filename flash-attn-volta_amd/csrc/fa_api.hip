@@ -537,7 +537,7 @@ int launch_dkdv(const fa::BwdArgs &a, hipStream_t stream) {
 template <typename E, int D, bool CAUSAL>
 int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
   const int64_t heads = (int64_t)a.B * a.H;
-  const NcFused nc = nc_fused(a.B, a.Sq, a.Sk, a.H, a.Hk, D, 1);
+  const NcFused nc = nc_fused(a.B, a.Sq, a.Sk, a.H, a.Hk, D, a.seg_n);
   const bool split = !CAUSAL && nc.on ? nc.q2 : dq_split2(D, CAUSAL, a.Sq, heads);
   // Eight waves sharing each K / V tile, as in the forward: D = 64 (256
   // queries, no key split) below two rounds ((1,4096,16) 235.7 us the
@@ -1513,12 +1513,13 @@ int run_dq(const void *dout, const void *q, const void *k, const void *v, const 
            const int64_t *k_st, const int64_t *v_st, const int64_t *dq_st, float sm_scale,
            int causal, void *stream, const void *o = nullptr, const int64_t *o_st = nullptr,
            unsigned *cnt_zero = nullptr, int n_cnt_zero = 0, int dq_split = 0,
-           float *dq_part = nullptr, float *rmax_out = nullptr) {
+           float *dq_part = nullptr, float *rmax_out = nullptr, int seg_n = 1) {
   const LaunchDevice launch_dev(stream);
   fa::BwdArgs a;
   int rc = dq_args(dout, q, k, v, lse, delta, dq, s, do_st, q_st, k_st, v_st, dq_st, sm_scale, o,
                    o_st, cnt_zero, n_cnt_zero, dq_split, dq_part, rmax_out, &a);
   if (rc) return rc;
+  a.seg_n = seg_n;   // the dK/dV launch's, for the layout rule
   hipStream_t st = static_cast<hipStream_t>(stream);
   FA_DISPATCH(launch_dq, s, causal, a, st);
 }
@@ -1623,7 +1624,8 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
   // stream, zeroes the key-block split's counters and leaves its split
   // query blocks' halves for the dK/dV kernel to add.
   if ((rc = run_dq(dout, q, k, v, lse, delta, dq, s, do_st, q_st, k_st, v_st, dq_st, sm_scale,
-                   causal, stream, o, o_st, cnt, (int)plan.slots, qplan.split, dq_part, rmax)))
+                   causal, stream, o, o_st, cnt, (int)plan.slots, qplan.split, dq_part, rmax,
+                   seg_n)))
     return rc;
   return run_dkdv(dout, q, k, v, lse, delta, rmax, dk, dv, s, do_st, q_st, k_st, v_st, dk_st,
                   dv_st, sm_scale, causal, stream, plan.split_kt, cnt, part, &qplan, dq_part, dq,

@@ -16,7 +16,7 @@ import torch
 
 from helpers import TOL, default_scale, max_abs
 from oracle import attention as orc
-from test_bwd_gpu import _bwd_capi
+from test_bwd_gpu import _bwd_capi, _bwd_three_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +82,21 @@ def test_noalloc_keeps_its_schedule():
     got = _call(lib, "fa_bwd_gqa_noalloc", do, q, k, v, o, lse, True)
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+def test_dq_layout_beside_segments():
+    """Segments that leave the fused launch leave its dQ layout too: dQ is then
+    bit for bit fa_bwd_dq's on the same heads ungrouped, whose grid takes the
+    same layout rule (208 blocks of 128 rows: key-split)."""
+    from flash_attn_volta import _capi, flash_attn_forward_gqa
+    B, S, H, Hk, D = 1, 1600, 16, 4, 128
+    print("[case] dQ layout beside segments", flush=True)
+    lib = _capi.load()
+    best = lib.fa_bwd_best_workspace_bytes(B, S, S, H, Hk, D, 0)
+    assert best > lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, Hk, D, 0), "segments must apply"
+    q, k, v, do = (t.cuda() for t in orc.make_inputs_gqa(B, S, S, H, Hk, D, seed=19, dtype=F16))
+    o, lse = flash_attn_forward_gqa(q, k, v, return_softmax_lse=True)
+    dq = _bwd_capi(do, q, k, v, o, lse, False, best, 0xFF)[0]
+    ke, ve = (t.repeat_interleave(H // Hk, dim=2).contiguous() for t in (k, v))
+    (ref, _, _), _ = _bwd_three_launches(do, q, ke, ve, o, lse, False, default_scale(D, None))
+    assert torch.equal(dq, ref)
