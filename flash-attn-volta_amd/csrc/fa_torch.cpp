@@ -103,22 +103,24 @@ bool aligned(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()
 
 // The kernels' strides of a (B, S, H, D) tensor they can read in place (unit
 // D stride, the others non-negative multiples of 8 elements, 128 rows of a
-// head within 31-bit byte offsets), 0 for size-1 dims, as the plan's; false
-// for any other layout.
-bool kernel_strides(const Tensor &t, int64_t (&st)[4]) {
+// head within 31-bit byte offsets; `half_cols`, the attention kernels at 16
+// columns: a whole head), 0 for size-1 dims, as the plan's; false for any
+// other layout.
+bool kernel_strides(const Tensor &t, int64_t (&st)[4], bool half_cols = false) {
   if (t.stride(3) != 1) return false;
   for (int i = 0; i < 3; ++i) {
     st[i] = t.size(i) == 1 ? 0 : t.stride(i);
     if (st[i] < 0 || st[i] % 8 != 0) return false;
   }
   st[3] = 1;
+  if (half_cols && st[1] > 0 && t.size(1) - 1 > (INT32_MAX - 64) / (2 * st[1])) return false;
   return st[1] <= (INT32_MAX - 2 * t.size(3)) / (2 * 127);
 }
 
 // `t` as the kernels read it, its strides in `st`: itself where the layout and
 // alignment allow, else a contiguous copy.
-Tensor kernel_ready(const Tensor &t, int64_t (&st)[4]) {
-  if (kernel_strides(t, st) && aligned(t)) return t;
+Tensor kernel_ready(const Tensor &t, int64_t (&st)[4], bool half_cols = false) {
+  if (kernel_strides(t, st, half_cols) && aligned(t)) return t;
   Tensor c = t.clone(at::MemoryFormat::Contiguous);
   kernel_strides(c, st);
   return c;
@@ -183,15 +185,16 @@ struct FlashAttnFn : public torch::autograd::Function<FlashAttnFn> {
     for (int i : {1, 2}) check_saved(s[i], {p.B, p.Sk, p.Hk, cols}, dtype, device);
     check_saved(s[4], {p.B, p.H, p.Sq}, at::kFloat, device);
     int64_t q_st[4], k_st[4], v_st[4], o_st[4], do_st[4];
-    const Tensor q = kernel_ready(s[0], q_st), k = kernel_ready(s[1], k_st),
-                 v = kernel_ready(s[2], v_st), out = kernel_ready(s[3], o_st);
+    const bool half = cols != p.D;
+    const Tensor q = kernel_ready(s[0], q_st, half), k = kernel_ready(s[1], k_st, half),
+                 v = kernel_ready(s[2], v_st, half), out = kernel_ready(s[3], o_st, half);
     const Tensor lse = s[4].is_contiguous() && aligned(s[4])
                            ? s[4] : s[4].clone(at::MemoryFormat::Contiguous);
     // dO as the kernels read it: the forward's dtype, in place when its
     // layout allows (a model's transposed (B, H, S, D) gradient does: making
     // it contiguous cost 11 us of 113 at (8,1024,12,64)), 16-byte aligned
     const Tensor dout = kernel_ready(
-        grads[0].scalar_type() == dtype ? grads[0] : grads[0].to(dtype), do_st);
+        grads[0].scalar_type() == dtype ? grads[0] : grads[0].to(dtype), do_st, half);
     Tensor dq = at::empty({p.B, p.Sq, p.H, cols}, q.options());
     // separate allocations, as the Python path's
     Tensor dk = at::empty({p.B, p.Sk, p.Hk, cols}, q.options());

@@ -70,10 +70,14 @@ def kernel_dims(D: int, dtype):
 
 def planned_dim(*tensors) -> bool:
     """The kernels take these (B, S, heads, D) tensors' head_dim without
-    padding: a native one, or 16 with heads of under 2^31 bytes."""
+    padding: a native one, or 16 with heads (and tiles of 128 rows) of under
+    2^31 bytes, in the tensors' own layouts and in the contiguous one of
+    their outputs and gradients."""
     D = tensors[0].size(3)
     return D in NATIVE_HEAD_DIMS or (D == 16 and all(
-        (t.size(1) - 1) * t.stride(1) * 2 + 64 < 2 ** 31 for t in tensors))
+        t.size(1) == 1 or
+        max(t.size(1) - 1, 127) * max(t.stride(1), t.size(2) * D) * 2 + 64 < 2 ** 31
+        for t in tensors))
 
 
 _STRIDES = {}
