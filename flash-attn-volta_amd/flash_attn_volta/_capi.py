@@ -14,7 +14,7 @@ import threading
 LIB_NAME = "libfa_mi355x.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 # status codes (enum fa_status)
 FA_OK = 0
@@ -189,10 +189,10 @@ def load(path: str | None = None):
                 f"{p} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
                 "(or flash_attn_volta.build.build_library()) first. There is no fallback path.")
         lib = ctypes.CDLL(p)
-        _declare(lib)
-        v = lib.fa_abi_version()
+        v = lib.fa_abi_version()        # before the symbols that another version may lack
         if v != ABI_VERSION:
             raise LibraryNotBuilt(f"{p} has ABI version {v}, expected {ABI_VERSION}; rebuild it")
+        _declare(lib)
         if path is None:
             _lib = lib
         return lib

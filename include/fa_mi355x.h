@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define FA_ABI_VERSION 9
+#define FA_ABI_VERSION 10
 
 /* Size of the static device scratch buffer that fa_bwd_gqa_noalloc uses as
  * its workspace (one per GPU, held for the life of the process). */

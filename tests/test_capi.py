@@ -46,7 +46,7 @@ def test_library_exports_every_declared_symbol(lib):
 
 
 def test_abi_version(lib):
-    assert lib.fa_abi_version() == _capi.ABI_VERSION == 9
+    assert lib.fa_abi_version() == _capi.ABI_VERSION == 10
 
 
 def test_noalloc_scratch_size_matches_header():
@@ -543,6 +543,17 @@ int fa_fwd_ws(void) { return -9; }
 int fa_bwd(void) { return -9; }
 int fa_bwd_gqa(void) { return -9; }
 """
+
+
+def test_loader_refuses_a_library_of_another_abi(tmp_path):
+    """A library of another ABI version is named as such, also where it lacks
+    entry points of this one."""
+    import subprocess
+    src, out = tmp_path / "stub.c", tmp_path / "libfa_mi355x.so"
+    src.write_text(_STUB_LIB % (_capi.ABI_VERSION - 1))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(out)], check=True)
+    with pytest.raises(_capi.LibraryNotBuilt, match=f"expected {_capi.ABI_VERSION}; rebuild it"):
+        _capi.load(str(out))
 
 
 def test_torch_node_refuses_a_library_of_another_abi(tmp_path):
