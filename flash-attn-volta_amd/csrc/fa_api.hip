@@ -1315,6 +1315,32 @@ size_t segment_bytes(const Shape &s) {
   return (size_t)2 * s.B * s.Hk * (size_t)s.Sk * s.D * sizeof(float);
 }
 
+// The shortest sweep (query tiles of the first key block, over its group) that
+// segments pay for on a causal grid of grouped heads filling `f` of a round:
+// their rows, the sum launch (2.5 us, all there is to gain on 14 us steps) and
+// the second round of segments that a grid past half a round starts.
+// Measured, the backward, us, whole / the segments below:
+//   D = 128: (5,56,64/8) (f 0.16, 8 tiles) 25 / 29, (6,37,64/8) (0.19, 8) 24 / 32,
+//     (6,191,16/4) (0.19, 12) 36 / 34, (3,540,16/8) (0.47, 18) 46 / 49,
+//     (2,834,16/8) (0.44, 28) 62 / 60, (4,440,64/8) (0.5, 56) 117 / 104,
+//     (6,380,32/8) (0.56, 24) 71 / 86, (3,719,32/8) (0.56, 48) 101 / 99, (8,555,28/4)
+//     (0.62, 63) 130 / 139, (7,649,32/4) (0.66, 88) 172 / 168, (3,951,16/8) (0.75, 30)
+//     72 / 89, (5,1028,32/4) (0.70, 136) 257 / 246, (7,951,28/4) (0.88, 105) 233 / 259,
+//     (1,3490,32/8) (0.88, 220) 424 / 383, (3,1247,32/8) (0.94, 80) 181 / 196,
+//     (2,2037,32/8) (1.0, 128) 271 / 291, (2,4022,16/4) (1.0, 252) 499 / 487;
+//   D = 64: (3,38,32/8) (f 0.05, 4 tiles) 14 / 17, (5,117,16/4) (0.04, 8) 18 / 16,
+//     (8,119,32/8) (0.13, 8) 19 / 20, (5,193,32/8) (0.16, 16) 27 / 26, (3,635,16/8)
+//     (0.23, 20) 30 / 30, (2,1621,16/8) (0.41, 52) 67 / 64, (6,585,32/8) (0.47, 40)
+//     61 / 68, (4,914,64/8) (0.5, 120) 162 / 153, (7,575,64/8) (0.55, 72) 112 / 123,
+//     (8,1356,28/4) (0.69, 154) 236 / 233;
+//   D = 32: (1,91,32/8) (0.02, 8) 14 / 17, (8,238,8/2) (0.06, 16) 20 / 18, (5,181,32/8)
+//     (0.16, 12) 21 / 22, (3,487,16/4) (0.09, 32) 30 / 21.
+double least_sweep(int D, double f) {
+  if (D >= 128) return f <= 0.45 ? 4.0 + 40.0 * f : 22.0 + 290.0 * (f - 0.45);
+  if (f > 0.41) return 50.0 + 330.0 * (f - 0.41);
+  return D == 64 ? 7.5 + 75.0 * (f > 0.06 ? f - 0.06 : 0.0) : 10.0 + 80.0 * f;
+}
+
 // Sweep segments of the dK/dV blocks (fa::BwdArgs::seg_n), given the room
 // (fa_bwd_best_workspace_bytes).  A key block's sweep covers every query
 // head of its group, so few key/value heads leave few, long workgroups:
@@ -1387,6 +1413,7 @@ int dkdv_segments(const Shape &s, int causal) {
     bwd_plans(s, causal, plan, qplan);
     return qplan.split == 0 ? 2 : 1;
   }
+  if ((double)sweep < least_sweep(s.D, (double)blocks / (double)slots)) return 1;
   int64_t n = (slots + blocks - 1) / blocks;
   if (n < 2 && sweep >= 192) n = 2;
   // short sweeps: fewer than fill every slot, of at least 8 tiles -- or, while

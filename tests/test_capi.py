@@ -207,6 +207,23 @@ def test_best_workspace_is_bounded(lib):
             lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, H, 128, 0)
 
 
+@pytest.mark.parametrize("B,S,H,Hk,D,segments", [
+    (3, 951, 16, 8, 128, False), (6, 380, 32, 8, 128, False), (6, 37, 64, 8, 128, False),
+    (7, 951, 28, 4, 128, False), (3, 1247, 32, 8, 128, False), (6, 191, 16, 4, 128, True),
+    (1, 4000, 28, 4, 128, True), (1, 3490, 32, 8, 128, True), (1, 128, 28, 4, 128, True),
+    (6, 585, 32, 8, 64, False), (7, 575, 64, 8, 64, False), (3, 38, 32, 8, 64, False),
+    (5, 117, 16, 4, 64, True), (8, 1356, 28, 4, 64, True), (1, 700, 14, 2, 64, True),
+    (1, 91, 32, 8, 32, False), (3, 487, 16, 4, 32, True)])
+def test_causal_segments_of_short_sweeps(lib, B, S, H, Hk, D, segments):
+    """Causal grids of grouped heads on both sides of the shortest sweep that
+    segments pay for (256 CUs without a GPU)."""
+    best = lib.fa_bwd_best_workspace_bytes(B, S, S, H, Hk, D, 1)
+    one, mini = 2 * B * Hk * S * D * 4, lib.fa_bwd_workspace_bytes(B, S, H, D)
+    assert ((best - mini) // one >= 2 and (best - mini) % one == 0) == segments
+    if not segments:
+        assert best == lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, Hk, D, 1)
+
+
 def test_bwd_validation(lib):
     assert _bwd(lib, ws=None) == _capi.FA_ERR_WORKSPACE
     assert _bwd(lib, ws_bytes=16) == _capi.FA_ERR_WORKSPACE
