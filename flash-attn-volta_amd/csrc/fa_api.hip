@@ -718,7 +718,8 @@ SplitPlan splitkv_plan(const Shape &s) {
 //     ((32, 1, 3001 keys, 32 heads / 8, 128) bf16: 222 us plain, 74 us
 //     packed, 5.3 TB/s, a large copy's rate; (64, 4, 4000, 32 / 8, 128)
 //     595 -> 179 us);
-//   * chunks: any short block of queries whose plain grid leaves CUs idle.
+//   * chunks: short blocks of queries whose plain grid leaves CUs idle or
+//     most of its tiles' rows empty.
 //     The model below prices both in us: a workgroup's 64 x 64 tile step
 //     takes `lone` alone on its CU and grows with the workgroups per CU
 //     from where they fill it; a workgroup's start-up; and for a split the
@@ -729,6 +730,19 @@ SplitPlan splitkv_plan(const Shape &s) {
 //     (1,1000,9000,14/2,64) 67 -> 48; against it (1,600,3000,32/8,128)
 //     44 -> 56, (1,300,2000,28/4,128) 27.5 -> 28.5 and (1,200,1000,32/32,128)
 //     16.0 -> 18.6 in two ranges, which the model leaves plain.
+//     D = 128 past a few heads is bound by reading K and V, once per 128-row
+//     tile in the plain layout and once per 64-row one here (7 TB/s on both
+//     sides) unless a head's tiles run together and share L2, which they do
+//     while all heads' next tiles fit beside them.  So not where the packed
+//     tiles are more and B * Hk is over 128, nor where they are half as many
+//     again on full grids: (50,70,10934,16/8) 707 / 1101, (31,74,7649,16/8) not
+//     causal 277 / 410, (32,70,4096,32/8) 313 / 373, (64,130,4096,28/4) 1056 / 1100,
+//     (23,205,12739,32/4) 1360 / 1746, (16,200,8448,32/8) 634 / 655; but
+//     (64,20,3000,32/8) 446 -> 326, (256,10,4096,64/8) 4584 -> 1719, (32,130,4096,
+//     16/1) 240 -> 188, (7,129,10210,32/8) 354 -> 210, not causal (22,77,3944,32/4)
+//     218 -> 152, (32,92,6392,32/4) 492 -> 451.
+//     The ranges' fp32 rows take at most 128 MiB, or a sixteenth of q, k, v
+//     and o ((256,10,4096,64/8): 161 MiB of 8512).
 SplitPlan fwd_split_plan(const Shape &s, int causal) {
   const SplitPlan none{0, 0};
   const int64_t grp = s.H / s.Hk;
@@ -743,6 +757,10 @@ SplitPlan fwd_split_plan(const Shape &s, int causal) {
   // half of the keys lie before the block)
   if (causal && (int64_t)s.Sk < 2 * (int64_t)s.Sq) return none;
   const double lone = s.D >= 128 ? 0.65 : 0.47, start = 6.0;
+  // (D = 128: two workgroups fill a CU, a third waits for a slot, so a step
+  // goes from 1.10 at two to 1.40 just above: 8448 keys, 32 / 8 heads, ranges
+  // that make two a CU or less against the next more: Sq = 256 49.0 (4) / 61.5
+  // (5), 288 56.5 (3) / 71.7 (4), 352 67.4 (2) / 88.1 (3))
   auto sweep_us = [&](int64_t wgs, int64_t tiles) {
     const double w = (double)wgs / (double)cus;   // workgroups per CU
     double step = lone;
@@ -754,15 +772,25 @@ SplitPlan fwd_split_plan(const Shape &s, int causal) {
     return step * (double)tiles + start;
   };
   const int64_t tiles = (s.Sk + 63) / 64, packed = packed_tiles(s);
-  // (D = 128, a head's K and V past an XCD's L2: the sweeps of a plain grid
-  // of one workgroup per CU or less, which share them only across a head's
-  // query tiles, drift apart and miss: 0.91 us a step at 17000 keys)
+  const int64_t heads = (int64_t)s.B * s.H;
+  const int64_t wide = grid128(s.Sq, heads);
+  if (s.D >= 128 && 100 * packed > 104 * wide &&
+      ((int64_t)s.B * s.Hk > 128 || (100 * packed > 155 * wide && wide >= 2 * cus)))
+    return none;
+  const double tensors = 4.0 * s.D * (heads * (double)s.Sq + (double)s.B * s.Hk * s.Sk);
+  const double room = tensors / 16 > 134217728.0 ? tensors / 16 : 134217728.0;
+  // (a plain grid of at most one workgroup per CU over more than 6 MB of a
+  // head's K and V: plain / two ranges (512,12500,32/8) 134 / 115, (512,17000)
+  // 180 / 152, (400,12500) 131 / 98.  The line could lie lower: the plain sweep
+  // takes 0.66 us a step on both sides of it, and (512,8448) is 92 / 82,
+  // (512,11500) 122 / 107, both left plain.)
   const double far =
       s.D >= 128 && plain <= cus && (double)s.Sk * s.D * 4.0 > 6.0e6 ? 1.4 : 1.0;
   double best = 0.88 * (far * (sweep_us(plain, tiles) - start) + start);
   int64_t best_n = 0;
   for (int64_t n = 2; n <= 32 && 4 * n <= tiles; ++n) {
     const double rows = (double)s.B * s.H * s.Sq * n;
+    if (rows * (s.D + 1) * 4.0 > room) break;
     const double c = sweep_us(packed * n, (tiles + n - 1) / n) + 2.0 + n +
                      rows * (s.D + 1) * 8.0 / 5.0e6;
     if (c < best) {

@@ -224,6 +224,30 @@ def test_causal_segments_of_short_sweeps(lib, B, S, H, Hk, D, segments):
         assert best == lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, Hk, D, 1)
 
 
+def test_forward_workspace_is_bounded(lib):
+    """Key ranges of the forward take at most 130 MiB of fp32 rows, or a
+    sixteenth of q, k, v and o; D = 128 grids whose 128-row tiles are fewer
+    than the packed 64-row ones run plain (256 CUs without a GPU)."""
+    most = 0
+    for B in (1, 4, 16, 37, 64, 256):
+        for Sq in (1, 8, 20, 64, 70, 130, 200, 512, 2048):
+            for Sk in (256, 3000, 8448, 32768):
+                for H, Hk in ((32, 8), (28, 4), (64, 8), (32, 4), (32, 32), (8, 1)):
+                    for D in (64, 128):
+                        for causal in (0, 1):
+                            n = lib.fa_fwd_workspace_bytes(B, Sq, Sk, H, Hk, D, causal)
+                            tensors = 4 * D * B * (H * Sq + Hk * Sk)
+                            assert n <= max(130 << 20, tensors // 16), (B, Sq, Sk, H, Hk, D)
+                            most = max(most, n)
+    assert most > 130 << 20
+    for B, Sq, Sk, H, Hk in ((32, 70, 4096, 32, 8), (50, 70, 10934, 16, 8), (23, 205, 12739, 32, 4),
+                             (64, 130, 4096, 28, 4), (256, 200, 8448, 64, 8)):
+        assert lib.fa_fwd_workspace_bytes(B, Sq, Sk, H, Hk, 128, 1) == 0
+    for B, Sq, Sk, H, Hk in ((64, 20, 3000, 32, 8), (256, 10, 4096, 64, 8), (7, 129, 10210, 32, 8),
+                             (1, 256, 8448, 32, 8), (32, 1, 3001, 28, 4)):
+        assert lib.fa_fwd_workspace_bytes(B, Sq, Sk, H, Hk, 128, 1) > 0
+
+
 def test_bwd_validation(lib):
     assert _bwd(lib, ws=None) == _capi.FA_ERR_WORKSPACE
     assert _bwd(lib, ws_bytes=16) == _capi.FA_ERR_WORKSPACE
