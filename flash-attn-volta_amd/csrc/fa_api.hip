@@ -1343,6 +1343,13 @@ size_t segment_bytes(const Shape &s) {
   return (size_t)2 * s.B * s.Hk * (size_t)s.Sk * s.D * sizeof(float);
 }
 
+// Workspace past delta and the maxima that selects `n` segments: their rows,
+// or just more than `splits`, the size that selects the splits.
+size_t segments_room(const Shape &s, int n, size_t splits) {
+  const size_t rows = (size_t)n * segment_bytes(s);
+  return rows > splits ? rows : splits + 256;
+}
+
 // The shortest sweep (query tiles of the first key block, over its group) that
 // segments pay for on a causal grid of grouped heads filling `f` of a round:
 // their rows, the sum launch (2.5 us, all there is to gain on 14 us steps) and
@@ -1630,10 +1637,12 @@ int run_bwd(const void *dout, const void *q, const void *k, const void *v, const
                                           delta_bytes(s.B, s.Sq, s.H));
   const size_t dbytes = delta_bytes(s.B, s.Sq, s.H) + rbytes;
   // Sweep segments where the workspace has room for all of them
-  // (fa_bwd_best_workspace_bytes), in place of both splits.
+  // (fa_bwd_best_workspace_bytes), in place of both splits -- not at the
+  // splits' own size, should that be enough.
+  const size_t splits = split_bytes(plan) + dq_split_bytes(qplan);
   int seg_n = dkdv_segments(s, causal);
-  if (workspace_bytes < dbytes + seg_n * segment_bytes(s)) seg_n = 1;
-  if (seg_n > 1 || workspace_bytes < dbytes + split_bytes(plan) + dq_split_bytes(qplan)) {
+  if (workspace_bytes < dbytes + segments_room(s, seg_n, splits)) seg_n = 1;
+  if (seg_n > 1 || workspace_bytes < dbytes + splits) {
     plan = DkdvSplit{};
     qplan = DqSplit{};
   }
@@ -2108,8 +2117,10 @@ size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, 
   const Shape s{B, Sq, Sk, H, Hk, D, FA_DTYPE_F16};
   if (check_shape(s) != FA_OK) return 0;
   const int seg_n = dkdv_segments(s, causal);
-  if (seg_n == 1) return fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, causal);
-  return delta_bytes(B, Sq, H) + rmax_bytes(B, Sq, H) + seg_n * segment_bytes(s);
+  const size_t both = fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, causal);
+  if (seg_n == 1) return both;
+  const size_t dbytes = delta_bytes(B, Sq, H) + rmax_bytes(B, Sq, H);
+  return dbytes + segments_room(s, seg_n, both - dbytes);
 }
 
 int fa_bwd(const void *dout, const void *q, const void *k, const void *v,
@@ -2159,7 +2170,7 @@ int fa_bwd_gqa_noalloc(const void *dout, const void *q, const void *k, const voi
     return FA_ERR_SCRATCH;
   void *ws = nullptr;
   if ((rc = scratch_for_stream(stream, &ws))) return rc;
-  // (the splits as fa_bwd_gqa with this size; no sweep segments)
+  // (the splits, as fa_bwd_gqa with this size; no sweep segments)
   const size_t most = fa_bwd_gqa_workspace_bytes(B, Sq, Sk, H, Hk, D, causal);
   return run_bwd(dout, q, k, v, o, lse, dq, dk, dv, ws,
                  most < FA_NOALLOC_SCRATCH_BYTES ? most : (size_t)FA_NOALLOC_SCRATCH_BYTES, s,

@@ -245,7 +245,8 @@ size_t fa_bwd_gqa_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, i
  * which fa_bwd / fa_bwd_gqa sweep every key block in segments, one
  * workgroup each: the fa_bwd_workspace_bytes minimum plus the segments'
  * fp32 dK and dV rows, at most 64 MiB, which a last launch adds in segment
- * order (0 on bad sizes).  Results differ from the other schedules' in rounding only and are
+ * order (or 256 bytes over fa_bwd_gqa_workspace_bytes, should the splits'
+ * size be larger; 0 on bad sizes).  Results differ from the other schedules' in rounding only and are
  * bit-reproducible.
  */
 size_t fa_bwd_best_workspace_bytes(int B, int Sq, int Sk, int H, int Hk, int D, int causal);

@@ -201,6 +201,10 @@ def test_best_workspace_is_bounded(lib):
                         assert blocks <= (256 if D == 128 else 512)
                         seen.add((D, causal, n))
     assert len(seen) > 20
+    # a size of its own also where the splits' is larger than the segments'
+    for B, S, H, Hk in ((1, 3776, 4, 2), (1, 3952, 4, 2), (2, 3776, 2, 1)):
+        assert lib.fa_bwd_best_workspace_bytes(B, S, S, H, Hk, 128, 1) > \
+            lib.fa_bwd_gqa_workspace_bytes(B, S, S, H, Hk, 128, 1)
     # the fused launch's own grids run whole sweeps
     for B, S, H in ((1, 3000, 12), (1, 4096, 4), (1, 1500, 8), (2, 1000, 10), (4, 1500, 6)):
         assert lib.fa_bwd_best_workspace_bytes(B, S, S, H, H, 128, 0) == \
