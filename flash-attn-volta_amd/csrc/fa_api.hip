@@ -223,10 +223,13 @@ int64_t grid128(int rows, int64_t heads) { return (int64_t)((rows + 127) / 128) 
 //   causal, D = 64: below 2.5 CUs' worth, and up to 4 on sweeps under 16
 //     tiles of 128 rows ((1,4096,20) 58 / 57, (1,4096,24) 67 / 61,
 //     (2,2048,25) 43 / 40, (1,4096,18) 53 / 55, (8,1024,12) 25 / 28,
-//     (5,1536,12) 32 / 37);
+//     (5,1536,12) 32 / 37; at the 2048 rows (1,1792,50) 36 / 41, (1,1920,48)
+//     35 / 40, (1,2048,44) 37 / 37, (1,2176,42) 41 / 39);
 //   causal, D = 128: below 2, and to 2.25 past 2048 rows ((1,3000,16) 47 / 56,
-//     (1,4096,16) 80 / 82, (1,2048,32) 49 / 45, (2,1024,32) 35 / 28, (1,4096,18)
-//     100 / 97, (1,4096,24) 125 / 112);
+//     (1,2560,26) 61 / 62, (1,3000,22) 68 / 71, (1,4096,16) 80 / 82, (1,2048,32)
+//     49 / 45, (2,1024,32) 35 / 28, (1,4096,18) 100 / 97, (1,4096,24) 125 / 112;
+//     the 2 to 2.25 also hold (1,2176,31) 70 / 55, (1,2304,29) 71 / 58 and
+//     (1,4096,17) 104 / 96, which no line here tells apart);
 //   not causal: D = 64 up to 2.5 ((1,4096,18) 94 / 103, (1,4096,20) 101 / 105,
 //     (1,4096,22) 119 / 108), D = 128 below one ((1,3800,8) 67 / 67, one
 //     round and more: launch_fwd).
@@ -441,7 +444,10 @@ int launch_fwd(const fa::FwdArgs &a, hipStream_t stream) {
   }
   if constexpr (!CAUSAL && D == 128) {
     // exactly one round of eight-wave key-split workgroups (128 queries
-    // each), long sweeps: (1,4096,8) 69 us, 72 unsplit; (1,4608,8) 131 / 109
+    // each), long sweeps: (1,4096,8) 69 us, 72 unsplit, (1,8192,4) 136 / 145;
+    // over a round (1,4224,8) 125 / 101, (1,4608,8) 131 / 109.  It wins on
+    // nearly full rounds too, left to the layouts below: (1,3712,8) 62 / 65,
+    // (1,3968,8) 69 / 72, (1,7936,4) 129 / 137
     if (grid128(a.Sq, heads) == device_cus() && a.Sk >= 2048)
       return launch_fwd_mode<E, D, CAUSAL, 2, 8>(a, stream);
   }
@@ -543,7 +549,9 @@ int launch_dq(const fa::BwdArgs &a, hipStream_t stream) {
   // queries, no key split) below two rounds ((1,4096,16) 235.7 us the
   // backward, 238.2 with four waves, (1,4096,30) 466 / 494, (1,4096,32) 466 /
   // 462, (4,4096,16) 947 / 924), D = 128 (128 queries, key split) on exactly
-  // one round ((1,4096,8) 234 / 239, (1,4096,14) 442 / 425).
+  // one round ((1,4096,8) 234 / 239, (1,4224,8) 402 / 372, (1,4096,14) 442 /
+  // 425; on nearly full ones it wins too: (1,3712,8) 209 / 215, (1,3968,8) 234 /
+  // 240).
   if constexpr (!CAUSAL && D == 64) {
     if (!split && eight_waves_64(a.Sq, a.Sk, heads) &&
         (int64_t)((a.Sq + 255) / 256) * heads < 2 * (int64_t)device_cus()) {

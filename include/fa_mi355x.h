@@ -431,6 +431,8 @@ int fa_rope_qk_fwd(const void *q, const void *k, void *q_out, void *k_out,
                    const int64_t q_out_strides[4], const int64_t k_out_strides[4],
                    const int64_t cs_strides[2], int dtype, void *stream);
 
+/* Or-ed into the dtype of fa_rope_qk_bwd: norm weight gradients in the element
+ * type (below). */
 #define FA_DW_16 0x200
 
 /* Bytes of workspace fa_rope_qk_bwd needs when a norm weight is given (0 for
