@@ -107,14 +107,15 @@ bool aligned(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()
 // columns: a whole head), 0 for size-1 dims, as the plan's; false for any
 // other layout.
 bool kernel_strides(const Tensor &t, int64_t (&st)[4], bool half_cols = false) {
-  if (t.stride(3) != 1) return false;
+  const int64_t *size = t.sizes().data(), *stride = t.strides().data();
+  if (stride[3] != 1) return false;
   for (int i = 0; i < 3; ++i) {
-    st[i] = t.size(i) == 1 ? 0 : t.stride(i);
-    if (st[i] < 0 || st[i] % 8 != 0) return false;
+    st[i] = size[i] == 1 ? 0 : stride[i];
+    if (st[i] < 0 || (st[i] & 7) != 0) return false;
   }
   st[3] = 1;
-  if (half_cols && st[1] > 0 && t.size(1) - 1 > (INT32_MAX - 64) / (2 * st[1])) return false;
-  return st[1] <= (INT32_MAX - 2 * t.size(3)) / (2 * 127);
+  if (half_cols && (double)(size[1] - 1) * st[1] * 2 + 64 > INT32_MAX) return false;
+  return 127 * st[1] * 2 + 2 * size[3] <= INT32_MAX;
 }
 
 // `t` as the kernels read it, its strides in `st`: itself where the layout and
