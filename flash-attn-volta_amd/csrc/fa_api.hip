@@ -464,6 +464,13 @@ int launch_pre(const fa::PreArgs &a, hipStream_t stream) {
   constexpr int RPB = 128;   // two lanes per row, 128 rows of one (b, h) per workgroup
   const int64_t grid = (int64_t)a.B * a.H * ((a.S + RPB - 1) / RPB);
   if (grid > 0x7fffffff) return FA_ERR_TOO_LARGE;
+  if constexpr (D == 32) {
+    if (a.cols == 16) {
+      hipLaunchKernelGGL((fa::fa_bwd_preprocess_kernel<E, 16>), dim3((unsigned)grid), dim3(256), 0,
+                         stream, a);
+      return launch_status();
+    }
+  }
   hipLaunchKernelGGL((fa::fa_bwd_preprocess_kernel<E, D>), dim3((unsigned)grid), dim3(256), 0,
                      stream, a);
   return launch_status();

@@ -186,7 +186,9 @@ struct PreArgs {
 // ulps of delta in dS, and which few depends on this order.)  With rmax
 // set, each wave also writes its 32 rows' group maxima (max |dO|, max
 // |delta|: BwdArgs::rmax), which maxima alone make exact whatever the order.
-template <typename E, int D>
+// COLS: the columns of a row (rows of 16 columns: an instance of its own, as
+// loads that depend on a run-time count do not all go out together).
+template <typename E, int COLS>
 __global__ __launch_bounds__(256) void fa_bwd_preprocess_kernel(PreArgs a) {
   constexpr int RPB = 128;   // rows per block, all of one (b, h)
   const int tid = threadIdx.x;
@@ -204,15 +206,14 @@ __global__ __launch_bounds__(256) void fa_bwd_preprocess_kernel(PreArgs a) {
     const int h = (int)(bh % a.H), b = (int)(bh / a.H);
     const f16 *po = a.o.head(b, h) + (int64_t)s * a.o.ss + 8 * g;
     const f16 *pg = a.dout.head(b, h) + (int64_t)s * a.dout.ss + 8 * g;
-    vec8<E> ov[D / 16], gv[D / 16];
+    vec8<E> ov[COLS / 16], gv[COLS / 16];
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-      const bool none = past_cols<D>(16 * c, a.cols);
-      ov[c] = none ? vec8<E>{} : ld8<E>(po + 16 * c);
-      gv[c] = none ? vec8<E>{} : ld8<E>(pg + 16 * c);
+    for (int c = 0; c < COLS / 16; ++c) {
+      ov[c] = ld8<E>(po + 16 * c);
+      gv[c] = ld8<E>(pg + 16 * c);
     }
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c)
+    for (int c = 0; c < COLS / 16; ++c)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         acc = __builtin_fmaf((float)ov[c][j], (float)gv[c][j], acc);
@@ -278,7 +279,7 @@ __device__ __forceinline__ void store_row(f16 *dst, const floatx16 (&acc)[D / 32
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       vec4<E> v4;
-      if (past_cols<D>(c_row(4 * r, g), cols)) continue;
+      if (past_cols<D>(c_row(4 * r, 0), cols)) continue;   // (the same for both g)
 #pragma unroll
       for (int j = 0; j < 4; ++j) v4[j] = (E)(acc[d][4 * r + j] * mul);
       *(vec4<E> *)(dst + 32 * d + c_row(4 * r, g)) = v4;
@@ -337,8 +338,7 @@ __device__ __forceinline__ void load_row_frags(vec8<E> (&f)[D / 16], const f16 *
                                                int row, int S, int g, int cols) {
   const f16 *p = head + (int64_t)min(row, S - 1) * ss + 8 * g;
 #pragma unroll
-  for (int c = 0; c < D / 16; ++c)
-    f[c] = past_cols<D>(16 * c, cols) ? vec8<E>{} : ld8<E>(p + 16 * c);
+  for (int c = 0; c < D / 16; ++c) f[c] = ld8_cols<E, D>(p, 16 * c, cols);
 }
 
 // ---------------------------------------------------------------------------

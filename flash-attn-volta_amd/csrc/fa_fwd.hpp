@@ -396,8 +396,7 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
     const f16 *qp = (SPLITKV ? a.q.head(b, hk * grp + qr % grp) + (int64_t)(qr / grp) * a.q.ss
                              : a.q.head(b, h) + (int64_t)qr * a.q.ss) + 8 * g;
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c)
-      qf[c] = past_cols<D>(16 * c, a.cols) ? vec8<E>{} : ld8<E>(qp + 16 * c);
+    for (int c = 0; c < D / 16; ++c) qf[c] = ld8_cols<E, D>(qp, 16 * c, a.cols);
     if (pre) {
 #pragma unroll
       for (int c = 0; c < D / 16; ++c)
@@ -814,7 +813,7 @@ __global__ __launch_bounds__(64 * NW) void fa_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         vec4<E> v4;
-        if (past_cols<D>(c_row(4 * r, g), a.cols)) continue;
+        if (past_cols<D>(c_row(4 * r, 0), a.cols)) continue;   // (the same for both g)
 #pragma unroll
         for (int j = 0; j < 4; ++j) v4[j] = (E)(oacc[d][4 * r + j] * inv);
         *(vec4<E> *)(orow + 32 * d + c_row(4 * r, g)) = v4;
